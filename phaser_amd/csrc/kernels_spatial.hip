@@ -457,11 +457,13 @@ __global__ void __launch_bounds__(256) k_spat_cross_zz(
         if (!entry(i, e, ii)) break;
         const float2 x = R[ii * ls + e];
         float2* a = &acc[ii * ls + e];
+        const bool sum = ((modes >> (2 * i)) & 3u) == 1u;
         if (first) {
-          *a = x;
+          // a NaN never has the largest energy: it only stays in a sum
+          const float en = x.x * x.x + x.y * x.y;
+          *a = sum || en == en ? x : make_float2(0.f, 0.f);
         } else {
           const float2 y = *a;
-          const bool sum = ((modes >> (2 * i)) & 3u) == 1u;
           const bool take = x.x * x.x + x.y * x.y > y.x * y.x + y.y * y.y;
           *a = sum ? cadd(y, x) : (take ? x : y);
         }

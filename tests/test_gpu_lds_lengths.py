@@ -96,3 +96,44 @@ def test_rotation_grid_against_oracle(po, B):
         corr, am = ctx.so3_correlate_coef(f.astype(np.complex64), h.astype(np.complex64))
     assert np.max(np.abs(corr - mag)) / mag.max() < 2e-4
     assert am == int(mag.argmax())
+
+
+@pytest.mark.parametrize("channels", [2, 4])
+def test_nan_channel_loses_the_fusion(channels):
+    """An intensity that is NaN at one point makes the packed intensity and
+    range spectra NaN; the fusion passes to a later channel, with two channels
+    to the absent ones' zero, in the fused pass as in the separate ones.  At
+    two voxels per axis no frequency is a mean of the channels, so that the
+    grid stays finite.  The sums of eight voxels differ by their order alone:
+    1e-5 of the largest entry."""
+    from phaser_amd.capi import Context, PhaserError
+    N, tgt, src = 2, _cloud(11), _cloud(12)
+    clouds = [tgt, src]
+    extra = [np.stack([c[:, 3] ** 2 / 100, 50 + c[:, 0]], 1).astype(np.float32) for c in clouds]
+    got = {}
+    with Context(bandwidth=4, n_voxels=N, max_points=6000, channels=channels) as ctx:
+        for i in range(len(tgt)):  # a point that no grid direction samples
+            bad = tgt.copy()
+            bad[i, 3] = np.nan
+            if np.isfinite(ctx.sample_s2(bad)).all():
+                break
+        d = [ctx.device_array(bad), ctx.device_array(src)]
+        e = [ctx.device_array(x) for x in extra]
+        ra = [a.ptr if channels == 4 else 0 for a in e]
+        grid = ctx.device_empty(N ** 3 * 4)
+        for occ in (1, -1):
+            ctx.set_tuning(occ_fwd=occ)
+            grid.upload(np.full(N ** 3, 7.0, np.float32))
+            try:
+                ctx.register_pairs_channels_device([d[0].ptr], ra[:1], [len(bad)], [d[1].ptr],
+                                                   ra[1:], [len(src)], d_trans=grid.ptr)
+            except PhaserError as err:  # two channels: no positive peak
+                print(f"{channels} channels, occ {occ}: {err}", flush=True)
+            got[occ] = grid.download((N ** 3,), np.float32)
+        for a in d + e + [grid]:
+            a.free()
+    print(got, flush=True)
+    assert np.isfinite(got[-1]).all()
+    assert np.abs(got[1] - got[-1]).max() <= 1e-5 * np.abs(got[-1]).max()
+    if channels == 2:
+        assert not got[-1].any()
