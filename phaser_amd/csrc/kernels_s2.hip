@@ -780,10 +780,10 @@ __global__ void k_nn(const float4* __restrict__ grid, const float* __restrict__ 
 // F[s][m][i] = (sqrt(2 pi)/n) sum_j x[i][j] e^{-2 pi i m j / n}, m < bw
 // (s2_semi_memo.c:156-177), for R rows (s, i) per workgroup: one twiddle and
 // its index serve R rows, and neighbouring rows (n is even) store 16 bytes.
+// R = 1 or even.
 template <int R>
 __global__ void k_phi_dft(const float* __restrict__ sig, int n, int rows, int bw,
                           const float2* __restrict__ tw, float2* __restrict__ F) {
-  static_assert(R % 2 == 0, "rows in pairs");
   const int r0 = blockIdx.x * R;
   extern __shared__ float2 t[];  // n twiddles, then n x R values
   float* x = (float*)(t + n);
@@ -811,12 +811,17 @@ __global__ void k_phi_dft(const float* __restrict__ sig, int n, int rows, int bw
       e += m;
       if (e >= n) e -= n;
     }
+    if constexpr (R == 1) {
+      const int s = r0 / n, i = r0 - s * n;
+      F[((int64_t)s * bw + m) * n + i] = make_float2(ar[0] * scale, ai[0] * scale);
+    } else {
 #pragma unroll
-    for (int q = 0; q < R; q += 2) {
-      if (r0 + q >= rows) break;
-      const int s = (r0 + q) / n, i = r0 + q - s * n;
-      *(float4*)(F + ((int64_t)s * bw + m) * n + i) = make_float4(
-          ar[q] * scale, ai[q] * scale, ar[q + 1] * scale, ai[q + 1] * scale);
+      for (int q = 0; q < R; q += 2) {
+        if (r0 + q >= rows) break;
+        const int s = (r0 + q) / n, i = r0 + q - s * n;
+        *(float4*)(F + ((int64_t)s * bw + m) * n + i) = make_float4(
+            ar[q] * scale, ai[q] * scale, ar[q + 1] * scale, ai[q + 1] * scale);
+      }
     }
   }
 }
@@ -1009,12 +1014,17 @@ void launch_fst(const float* sig, int S, int bw, const float* legendre, const in
   // LDS reads) than multiply-adds, so a workgroup takes several rows or signals
   // where enough are left to fill the device.  Four rows against two: 256 grids
   // of 128^2 65.5 -> 60.5 us for both passes, 32 of 256^2 67.4 -> 62.6, the same
-  // at 8448 rows of 128; eight no better.  Two signals against one: 256 at
-  // bandwidth 64 60.5 -> 57.3, 64 at 96 65.0 -> 56.1, the same at 6144 sums and
-  // fewer at bandwidths 48 and 128.  One row and one signal: 86 and, at 96, 91;
-  // 4 grids at 64 / 160 20.4 / 60 against 18.3 / 46.
+  // at 8448 rows of 128; eight no better.  Two rows against one, whole calls of
+  // phz_s2_transform by samples (rows n): 300 x 300, 4 grids 153 against 156 us;
+  // 256 x 256, 8 187 / 194; 192 x 192, 8 127 / 129; 150 x 150, 16 134 / 137; the
+  // same at 256 K (128 x 128, 16 107); fewer lose: 192 x 192, 2 60.2 / 59.4;
+  // 150 x 150, 1 47.1 / 46.1; 96 x 96, 2 42.8 / 41.2.  Two signals against one:
+  // 256 at bandwidth 64 60.5 -> 57.3, 64 at 96 65.0 -> 56.1, the same at 6144
+  // sums and fewer at bandwidths 48 and 128.  Without the unrolled sums the
+  // same calls take 5 to 30 us more.
   if (rows >= 8192) dft(k_phi_dft<4>, 4);
-  else dft(k_phi_dft<2>, 2);
+  else if (rows * n >= 1 << 18) dft(k_phi_dft<2>, 2);
+  else dft(k_phi_dft<1>, 1);
   if (precision == 1) {
     launch_legendre_mfma(F, S, bw, legendre, leg_off_dev, coef, s);
     return;
