@@ -169,6 +169,9 @@ struct phz_ctx {
   GatherEntry* d_gather = nullptr;
   hipEvent_t gather_done = nullptr;
   bool gather_pending = false;
+  // a call that uses the accumulators (clear_accumulators) has begun and has
+  // not come to its end
+  bool accumulators_in_use = false;
   std::vector<void*> allocs;
   size_t alloc_bytes = 0;
   // per-stage HIP event timing (phz_set_profiling)
@@ -406,6 +409,55 @@ int check_config(const phz_config& cf) {
   return 0;
 }
 
+// sizes of the accumulators
+size_t cell_words(const phz_ctx* c) {
+  return (size_t)c->max_clouds * ((size_t)c->n * c->n + 6 * (size_t)c->n);
+}
+size_t sum_clouds(const phz_ctx* c) { return c->max_clouds > 16 ? c->max_clouds : 16; }
+size_t row_occ_bytes(const phz_ctx* c) {
+  return ((size_t)c->max_clouds * c->N * c->N + 3) / 4 * 4;
+}
+size_t plane_occ_bytes(const phz_ctx* c) { return ((size_t)c->max_clouds * c->N + 3) / 4 * 4; }
+
+// Zeroes the cell counts and band accumulators and the voxel accumulators.
+// They stay zero between calls: every pipeline run clears exactly what it
+// touched.
+int clear_accumulators(phz_ctx* c, hipStream_t s) {
+  const size_t voxels = (size_t)c->max_clouds * c->T3;
+  launch_fill_u32((uint32_t*)c->cells.cell_count, cell_words(c), 0u, s);
+  launch_fill_u32((uint32_t*)c->d_sumI, sum_clouds(c) * c->T3, 0u, s);
+  launch_fill_u32((uint32_t*)c->d_sumR, voxels, 0u, s);
+  launch_fill_u32(c->d_cnt, voxels, 0u, s);
+  launch_fill_u32((uint32_t*)c->d_row_occ, row_occ_bytes(c) / 4, 0u, s);
+  launch_fill_u32((uint32_t*)c->d_plane_occ, plane_occ_bytes(c) / 4, 0u, s);
+  if (c->cfg.channels == 4) {
+    launch_fill_u32((uint32_t*)c->d_sumF, voxels, 0u, s);
+    launch_fill_u32((uint32_t*)c->d_sumA, voxels, 0u, s);
+  }
+  PHZ_HIP(hipGetLastError());
+  return 0;
+}
+
+// A call's use of the accumulators on stream s: one that returns between
+// begin() and end() may have queued a part of its kernels only, so it waits
+// for those, and the next call clears what they left (counts that do not
+// start from zero would send points past the end of their cloud).
+struct AccumulatorUse {
+  phz_ctx* c;
+  hipStream_t s;
+  AccumulatorUse(phz_ctx* c_, hipStream_t s_) : c(c_), s(s_) {}
+  ~AccumulatorUse() {
+    if (c->accumulators_in_use) (void)hipStreamSynchronize(s);
+  }
+  int begin() {
+    if (c->accumulators_in_use) TRY(clear_accumulators(c, s));
+    c->accumulators_in_use = true;
+    return 0;
+  }
+  // the stream is idle after the call's last kernel
+  void end() { c->accumulators_in_use = false; }
+};
+
 int init_ctx(phz_ctx* c) {
   const phz_config& cf = c->cfg;
   TRY(check_config(cf));
@@ -508,8 +560,7 @@ int init_ctx(phz_ctx* c) {
   c->cells.pts = c->d_pts;
   TRY(dalloc(c, &c->d_npts, (size_t)M));
   TRY(dalloc(c, &c->d_gather, (size_t)M));
-  const size_t cell_words = (size_t)M * (nq + 6 * c->n);
-  TRY(dalloc(c, &c->cells.cell_count, cell_words));
+  TRY(dalloc(c, &c->cells.cell_count, cell_words(c)));
   c->cells.band_th = (unsigned*)(c->cells.cell_count + (size_t)M * nq);
   c->cells.band_count = (int*)(c->cells.band_th + (size_t)M * 2 * c->n);
   c->cells.band_range = c->cells.band_th + (size_t)M * 3 * c->n;
@@ -544,14 +595,11 @@ int init_ctx(phz_ctx* c) {
   c->partials_per_pair = std::max(so3_gamma_blocks(c->Bo), spatial_c2r_blocks(c->Np));
   TRY(dalloc(c, &c->d_partials, (size_t)P * c->partials_per_pair));
   TRY(dalloc(c, &c->d_pose, (size_t)P));
-  const int MV = M > 16 ? M : 16;
-  TRY(dalloc(c, &c->d_sumI, (size_t)MV * c->T3));
+  TRY(dalloc(c, &c->d_sumI, sum_clouds(c) * c->T3));
   TRY(dalloc(c, &c->d_sumR, (size_t)M * c->T3));
   TRY(dalloc(c, &c->d_cnt, (size_t)M * c->T3));
-  const size_t occ_row_bytes = ((size_t)M * c->N * c->N + 3) / 4 * 4;
-  const size_t occ_plane_bytes = ((size_t)M * c->N + 3) / 4 * 4;
-  TRY(dalloc(c, &c->d_row_occ, occ_row_bytes));
-  TRY(dalloc(c, &c->d_plane_occ, occ_plane_bytes));
+  TRY(dalloc(c, &c->d_row_occ, row_occ_bytes(c)));
+  TRY(dalloc(c, &c->d_plane_occ, plane_occ_bytes(c)));
   TRY(dalloc(c, &c->d_spec, (size_t)(2 * M > 16 ? 2 * M : 16) * c->H));
   TRY(dalloc(c, &c->d_work, (size_t)P * c->H));
   TRY(dalloc(c, &c->d_corr_trans, (size_t)c->T3p));
@@ -571,18 +619,7 @@ int init_ctx(phz_ctx* c) {
   PHZ_HIP(hipHostMalloc((void**)&c->h_pose, sizeof(DevPose) * P, hipHostMallocDefault));
   PHZ_HIP(hipHostMalloc((void**)&c->h_gather, sizeof(GatherEntry) * M, hipHostMallocDefault));
   PHZ_HIP(hipEventCreateWithFlags(&c->gather_done, hipEventDisableTiming));
-  // the cell counts and band accumulators stay zero between calls, and so do
-  // the voxel accumulators: every pipeline run clears exactly what it touched
-  launch_fill_u32((uint32_t*)c->cells.cell_count, cell_words, 0u, c->stream);
-  launch_fill_u32((uint32_t*)c->d_sumI, (size_t)MV * c->T3, 0u, c->stream);
-  launch_fill_u32((uint32_t*)c->d_sumR, (size_t)M * c->T3, 0u, c->stream);
-  launch_fill_u32(c->d_cnt, (size_t)M * c->T3, 0u, c->stream);
-  launch_fill_u32((uint32_t*)c->d_row_occ, occ_row_bytes / 4, 0u, c->stream);
-  launch_fill_u32((uint32_t*)c->d_plane_occ, occ_plane_bytes / 4, 0u, c->stream);
-  if (cf.channels == 4) {
-    launch_fill_u32((uint32_t*)c->d_sumF, (size_t)M * c->T3, 0u, c->stream);
-    launch_fill_u32((uint32_t*)c->d_sumA, (size_t)M * c->T3, 0u, c->stream);
-  }
+  TRY(clear_accumulators(c, c->stream));
   PHZ_HIP(hipStreamSynchronize(c->stream));
   PHZ_CHECK(c->alloc_bytes == context_bytes(cf), "internal error: device memory estimate is stale");
   // the register engine from the start wherever it has the length: measured
@@ -967,9 +1004,10 @@ void to_result(const DevPose& d, phz_result* r) {
   r->reserved = 0;
 }
 
-int fetch_results(phz_ctx* c, int np, phz_result* out, hipStream_t s) {
+int fetch_results(phz_ctx* c, int np, phz_result* out, AccumulatorUse* use) {
   const DevPose* hp = c->h_pose;  // written by the last kernel
-  PHZ_HIP(hipStreamSynchronize(s));
+  PHZ_HIP(hipStreamSynchronize(use->s));
+  use->end();
   collect_timings(c);
   for (int p = 0; p < np; ++p) to_result(hp[p], &out[p]);
   // the reference's CHECKs on the peak windows (its process aborts there):
@@ -1158,12 +1196,14 @@ int phz_register_channels(phz_ctx* c, const float* target, const float* target_r
   TRY(load_cloud(c, 0, target, Pt, hipMemcpyHostToDevice, s, target_ra));
   TRY(load_cloud(c, 1, source, Ps, hipMemcpyHostToDevice, s, source_ra));
   TRY(commit_counts(c, 2, s));
+  AccumulatorUse use(c, s);
+  TRY(use.begin());
   TRY(exec_pairs(c, 1, false, s, rot_corr ? c->d_corr_rot : nullptr,
                  trans_corr ? c->d_corr_trans : nullptr));
   if (registered && Ps > 0) launch_apply_pose(c->d_pts + c->cap, Ps, c->d_pose, c->d_reg, s);
   // -4 (a failed peak-window check) still fills every output: the grids and
   // the registered cloud are copied before the status is returned
-  const int rc = fetch_results(c, 1, result, s);
+  const int rc = fetch_results(c, 1, result, &use);
   if (rc && rc != -4) return rc;
   const std::string pair_msg = g_last_error;
   const int64_t n3 = (int64_t)c->no * c->no * c->no;
@@ -1217,8 +1257,10 @@ int phz_register_pairs_channels_device(phz_ctx* c, int n, int shared_target,
       TRY(load_cloud(c, i, pts[i], counts[i], hipMemcpyDeviceToDevice, s, extra[i]));
     TRY(commit_counts(c, nt + n, s));
   }
+  AccumulatorUse use(c, s);
+  TRY(use.begin());
   TRY(exec_pairs(c, n, shared_target != 0, s, d_rot_corr, d_trans_corr));
-  return fetch_results(c, n, results, s);
+  return fetch_results(c, n, results, &use);
 }
 
 int phz_register_pairs(phz_ctx* c, int n, int shared_target, const float* const* targets,
@@ -1232,8 +1274,10 @@ int phz_register_pairs(phz_ctx* c, int n, int shared_target, const float* const*
   for (int p = 0; p < n; ++p)
     TRY(load_cloud(c, nt + p, sources[p], Ps[p], hipMemcpyHostToDevice, s));
   TRY(commit_counts(c, nt + n, s));
+  AccumulatorUse use(c, s);
+  TRY(use.begin());
   TRY(exec_pairs(c, n, shared_target != 0, s, nullptr, nullptr));
-  return fetch_results(c, n, results, s);
+  return fetch_results(c, n, results, &use);
 }
 
 int phz_memory_usage(const phz_ctx* c, size_t* bytes) {
@@ -1263,10 +1307,12 @@ int phz_register_device(phz_ctx* c, const float* d_target, int64_t Pt, const flo
     TRY(load_cloud(c, 1, d_source, Ps, hipMemcpyDeviceToDevice, s));
     TRY(commit_counts(c, 2, s));
   }
+  AccumulatorUse use(c, s);
+  TRY(use.begin());
   TRY(exec_pairs(c, 1, false, s, d_rot_corr, d_trans_corr));
   if (d_registered && Ps > 0)
     launch_apply_pose(c->d_pts + c->cap, Ps, c->d_pose, (float4*)d_registered, s);
-  return fetch_results(c, 1, result, s);
+  return fetch_results(c, 1, result, &use);
 }
 
 // ---------------------------------------------------------------- stages
@@ -1275,12 +1321,15 @@ int phz_sample_s2(phz_ctx* c, const float* pts, int64_t P, float* grids) {
   hipStream_t s = c->stream;
   TRY(load_cloud(c, 0, pts, P, hipMemcpyHostToDevice, s));
   TRY(commit_counts(c, 1, s));
+  AccumulatorUse use(c, s);
+  TRY(use.begin());
   launch_sample_s2(c->d_pts, c->d_npts, c->cap, 1, c->n, c->d_grid, c->d_theta, c->max_sq,
                    c->cells, c->d_grids, s);
   PHZ_HIP(hipGetLastError());
   PHZ_HIP(hipMemcpyAsync(grids, c->d_grids, sizeof(float) * 2 * c->n * c->n,
                          hipMemcpyDeviceToHost, s));
   PHZ_HIP(hipStreamSynchronize(s));
+  use.end();
   return 0;
 }
 
@@ -1358,6 +1407,8 @@ int phz_voxelize(phz_ctx* c, const float* pts, int64_t P, float* out, float* cou
   hipStream_t s = c->stream;
   TRY(load_cloud(c, 0, pts, P, hipMemcpyHostToDevice, s));
   TRY(commit_counts(c, 1, s));
+  AccumulatorUse use(c, s);
+  TRY(use.begin());
   launch_voxel_scatter(c->d_pts, c->d_npts, c->cap, 1, nullptr, 0, c->N, c->d_edges, c->d_sumI,
                        c->d_sumR, c->d_cnt, occ_from(c), s);
   PHZ_HIP(hipGetLastError());
@@ -1368,7 +1419,9 @@ int phz_voxelize(phz_ctx* c, const float* pts, int64_t P, float* out, float* cou
   PHZ_HIP(hipMemcpyAsync(k.data(), c->d_cnt, sizeof(uint32_t) * c->T3, hipMemcpyDeviceToHost, s));
   launch_voxel_clear(c->d_pts, c->d_npts, c->cap, 1, nullptr, 0, c->N, c->d_edges, c->d_sumI,
                      c->d_sumR, c->d_cnt, occ_from(c), s);
+  PHZ_HIP(hipGetLastError());
   PHZ_HIP(hipStreamSynchronize(s));
+  use.end();
   for (int64_t v = 0; v < c->T3; ++v) {
     out[v] = k[v] ? sI[v] / (float)k[v] : 0.f;
     out[c->T3 + v] = k[v] ? sR[v] / (float)k[v] : 0.f;
@@ -1383,6 +1436,8 @@ int phz_spatial_correlate(phz_ctx* c, int C, const float* f, const float* g, flo
   PHZ_CHECK(C >= 2 && C <= 8, "channel count must be in [2, 8]");
   hipStream_t s = c->stream;
   const int64_t T = c->T3, H = c->H;
+  AccumulatorUse use(c, s);
+  TRY(use.begin());
   PHZ_HIP(hipMemcpyAsync(c->d_sumI, f, sizeof(float) * C * T, hipMemcpyHostToDevice, s));
   PHZ_HIP(hipMemcpyAsync(c->d_sumI + C * T, g, sizeof(float) * C * T, hipMemcpyHostToDevice, s));
   launch_spatial_forward_dense(c->N, 2 * C, c->d_sumI, c->plan_N, c->d_tw_N, c->d_spec, c->tiles,
@@ -1412,6 +1467,7 @@ int phz_spatial_correlate(phz_ctx* c, int C, const float* f, const float* g, flo
   unsigned long long key = 0;
   PHZ_HIP(hipMemcpyAsync(&key, c->d_keys, sizeof(key), hipMemcpyDeviceToHost, s));
   PHZ_HIP(hipStreamSynchronize(s));
+  use.end();
   if (argmax) *argmax = key_index(key);
   if (corr) TRY(copy_sync(c, corr, c->d_corr_trans, sizeof(float) * c->T3p, hipMemcpyDeviceToHost));
   return 0;

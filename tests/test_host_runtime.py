@@ -1,0 +1,96 @@
+"""The host code of the library without a GPU: over a stand-in of the HIP
+runtime (tests/cpp/fake_hip.cc) that logs the launches and runs none, each
+scenario in a process of its own."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+import host_runtime
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("fake_hip") / "libamdhip64.so.7")
+    host_runtime.build(path)
+    return path
+
+
+def _run(fake, scenario, *args):
+    code = (f"import sys; sys.path.insert(0, {os.path.dirname(__file__)!r})\n"
+            "import test_host_runtime as t, host_runtime as h\n"
+            f"t.{scenario}(h.FakeHip({fake!r}), *{args!r})\nprint('scenario ok')\n")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0 and "scenario ok" in r.stdout, r.stdout + r.stderr
+
+
+
+
+def failed_launch(hip, kernel, call):
+    """A launch that fails inside a call: the call reports it and waits for
+    what it has queued; the next call clears the accumulators before any
+    kernel counts into them; the one after it clears nothing."""
+    import numpy as np
+    from phaser_amd.capi import Context, PhaserError
+    cloud = np.ones((40, 4), np.float32)
+
+    def go(ctx):
+        if call == "register":
+            ctx.register(cloud, cloud)
+        elif call == "graph":
+            ctx.set_graphs(True)
+            ctx.register(cloud, cloud)
+        elif call == "pairs":
+            ctx.register_pairs([cloud, cloud], [cloud, cloud])
+        elif call == "device":
+            a = [ctx.device_array(cloud) for _ in range(2)]
+            ctx.register_pairs_device([a[0].ptr], [40], [a[1].ptr], [40])
+        elif call == "sample":
+            ctx.sample_s2(cloud)
+        elif call == "voxelize":
+            ctx.voxelize(cloud)
+        else:
+            ctx.spatial_correlate(np.ones((2, 8 ** 3)), np.ones((2, 8 ** 3)))
+
+    def counts(log):
+        return host_runtime.launches(log, "k_project", "k_voxel_scatter", "k_spat_r2c", "graph")
+
+    with Context(bandwidth=8, n_voxels=8, max_points=64, max_batch=2, channels=4) as ctx:
+        hip.reset()
+        try:
+            go(ctx)
+        except PhaserError as e:  # no kernel ran: the peak windows hold zeros
+            assert "error -4" in str(e), e
+        usual = hip.log()
+        assert host_runtime.launches(usual, kernel), usual
+        hip.reset()
+        if call == "graph":
+            ctx.set_graphs(False)  # captured before: capture again
+        hip.fail(kernel)
+        with pytest.raises(PhaserError, match="an error"):
+            go(ctx)
+        log = hip.log()
+        at = [i for i, l in enumerate(log) if l == "failed"]
+        assert at and "wait" in log[at[0]:], log
+        fills = len(host_runtime.launches(usual, "k_fill_u32"))
+        for cleared in (8, 0):  # the accumulators of four channels
+            hip.reset()
+            try:
+                go(ctx)
+            except PhaserError as e:
+                assert "error -4" in str(e), e
+            log = hip.log()
+            first = counts(log)[0]
+            fill = host_runtime.launches(log, "k_fill_u32")
+            assert len(fill) == fills + cleared, log
+            assert len([i for i in fill if i < first]) >= cleared, log
+
+
+@pytest.mark.parametrize("kernel,call", [
+    ("k_cell_bands", "register"), ("k_cell_scatter", "register"), ("k_voxel_scatter", "register"),
+    ("k_trans_pose", "pairs"), ("k_cell_bands", "pairs"), ("k_cell_scatter", "device"),
+    ("k_cell_bands", "graph"), ("k_cell_scatter", "sample"), ("k_voxel_scatter", "voxelize"),
+    ("k_spat_cross_z", "spatial")])
+def test_accumulators_are_cleared_after_a_failed_call(fake, kernel, call):
+    _run(fake, "failed_launch", kernel, call)
