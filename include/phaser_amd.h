@@ -346,8 +346,8 @@ int phz_zscore_peaks(phz_ctx* ctx, const float* corr, int64_t n, const phz_zscor
  * Stockham kernel (limited by LDS; the tile never changes a line's
  * arithmetic, so these give bit-identical results), or 1 for the register
  * four-step kernel (n = 48 to 256 with factors 2, 3 and 5 as listed in
- * fft_reg.hpp; same transform, other rounding), which a new context uses
- * wherever it has the length, as phz_set_tuning does for 0. */
+ * fft_reg.hpp; same transform, other rounding), the default wherever it has
+ * the length.  A field of 0 is always what a new context has. */
 typedef struct {
   int32_t fwd_x, fwd_z, inv_x;   /* 0 = default */
   int32_t plane_fwd;   /* first forward pass on whole z planes in LDS (N <= 128):
@@ -357,11 +357,11 @@ typedef struct {
                           queries: 8 for the fewest, 1 or 2 for the most); exact
                           for every value */
   int32_t fused_reg;   /* the r2c, cross-spectrum and c2r passes on the register
-                          four-step kernels (the engine's lengths): 1 = on (as a
-                          new context is), 0/-1 = off */
+                          four-step kernels (the engine's lengths): 0 or 1 = on
+                          (default), -1 = off */
   int32_t so3_reg;     /* the SO(3) alpha and gamma passes on the register kernels
-                          (the engine's lengths, and n = 288, 300, 320): 1 = on (as
-                          a new context is), 0/-1 = off */
+                          (the engine's lengths, and n = 250, 288, 300, 320): 0 or
+                          1 = on (default), -1 = off */
   int32_t occ_fwd;     /* with fused_reg and the register engine for the forward
                           z pass: that pass runs inside the cross-spectrum
                           kernel (its output is never stored), and with the

@@ -409,6 +409,40 @@ int check_config(const phz_config& cf) {
   return 0;
 }
 
+// A field of 0 is what a new context has.  The register engine wherever it has
+// the length: against the LDS passes, whole calls at B = 64, 128^3 voxels, 16
+// pairs 1.03 against 3.44 ms, one pair 0.32 against 0.44 ms.  No whole-plane
+// forward pass: slower at N = 128 (one workgroup per CU).
+void apply_tuning(phz_ctx* c, const phz_tuning& t) {
+  c->tuning = t;
+  c->tiles.fwd_x = fft_cols_tile_ok(c->N, t.fwd_x) ? t.fwd_x : 0;
+  c->tiles.fwd_z = fft_cols_tile_ok(c->N, t.fwd_z) ? t.fwd_z : 0;
+  c->tiles.inv_x = fft_cols_tile_ok(c->N, t.inv_x) ? t.inv_x : 0;
+  c->tuning.fwd_x = c->tiles.fwd_x ? c->tiles.fwd_x : fft_cols_default_tile(c->N);
+  c->tuning.fwd_z = c->tiles.fwd_z ? c->tiles.fwd_z : fft_cols_default_tile(c->N);
+  c->tuning.inv_x = c->tiles.inv_x ? c->tiles.inv_x : fft_cols_default_tile(c->N);
+  c->plane_fwd = t.plane_fwd > 0 && spatial_plane_ok(c->N);
+  c->tuning.plane_fwd = c->plane_fwd ? 1 : -1;
+  c->tuning.nn_lanes = (t.nn_lanes == 1 || t.nn_lanes == 2 || t.nn_lanes == 4 ||
+                        t.nn_lanes == 8 || t.nn_lanes == 16)
+                           ? t.nn_lanes
+                           : 0;
+  c->tiles.fused_reg = t.fused_reg >= 0 && spatial_reg(c->N);
+  c->tuning.fused_reg = c->tiles.fused_reg ? 1 : -1;
+  c->so3_reg = t.so3_reg >= 0 && so3_reg_ok(c->Bo);
+  c->tuning.so3_reg = c->so3_reg ? 1 : -1;
+  c->occ_fwd = t.occ_fwd >= 0;
+  c->tuning.occ_fwd = c->occ_fwd ? 1 : -1;
+  c->inv_plane = t.inv_plane >= 0;
+  c->tuning.inv_plane = c->inv_plane ? 1 : -1;
+  c->nn_xcd = t.nn_xcd == 0 ? kNnXcdDefault : t.nn_xcd > 0;
+  c->tuning.nn_xcd = c->nn_xcd ? 1 : -1;
+  c->nn_seed = t.nn_seed == 0 ? kNnSeedDefault : (t.nn_seed > 0 ? (t.nn_seed & 3) : 0);
+  c->tuning.nn_seed = c->nn_seed ? c->nn_seed : -1;
+  c->xz_slab = t.xz_slab > 0;
+  c->tuning.xz_slab = c->xz_slab ? 1 : -1;
+}
+
 // sizes of the accumulators
 size_t cell_words(const phz_ctx* c) {
   return (size_t)c->max_clouds * ((size_t)c->n * c->n + 6 * (size_t)c->n);
@@ -622,29 +656,7 @@ int init_ctx(phz_ctx* c) {
   TRY(clear_accumulators(c, c->stream));
   PHZ_HIP(hipStreamSynchronize(c->stream));
   PHZ_CHECK(c->alloc_bytes == context_bytes(cf), "internal error: device memory estimate is stale");
-  // the register engine from the start wherever it has the length: measured
-  // against the LDS passes at B = 64, 128^3 voxels, 16 pairs 1.03 against
-  // 3.44 ms, one pair 0.32 against 0.44 ms; phz_autotune times both
-  c->tiles = spatial_default_tiles(c->N);
-  c->tuning.fwd_x = c->tiles.fwd_x;
-  c->tuning.fwd_z = c->tiles.fwd_z;
-  c->tuning.inv_x = c->tiles.inv_x;
-  c->plane_fwd = false;  // measured slower at N = 128 (one workgroup per CU)
-  c->tuning.plane_fwd = -1;
-  c->tuning.nn_lanes = 0;  // automatic, by clouds per launch
-  c->tuning.fused_reg = c->tiles.fused_reg ? 1 : -1;
-  c->so3_reg = so3_reg_ok(c->Bo);
-  c->tuning.so3_reg = c->so3_reg ? 1 : -1;
-  c->occ_fwd = true;
-  c->tuning.occ_fwd = 1;
-  c->inv_plane = true;
-  c->tuning.inv_plane = 1;
-  c->nn_xcd = kNnXcdDefault;
-  c->tuning.nn_xcd = kNnXcdDefault ? 1 : -1;
-  c->nn_seed = kNnSeedDefault;
-  c->tuning.nn_seed = kNnSeedDefault ? kNnSeedDefault : -1;
-  c->xz_slab = false;
-  c->tuning.xz_slab = -1;
+  apply_tuning(c, phz_tuning{});
   return 0;
 }
 
@@ -1817,36 +1829,6 @@ int phz_memcpy(phz_ctx* c, void* dst, const void* src, size_t bytes, int kind) {
   PHZ_HIP(hipStreamSynchronize(c->stream));
   TRY(copy_sync(c, dst, src, bytes, k[kind]));
   return 0;
-}
-
-static void apply_tuning(phz_ctx* c, const phz_tuning& t) {
-  c->tuning = t;
-  c->tiles.fwd_x = fft_cols_tile_ok(c->N, t.fwd_x) ? t.fwd_x : 0;
-  c->tiles.fwd_z = fft_cols_tile_ok(c->N, t.fwd_z) ? t.fwd_z : 0;
-  c->tiles.inv_x = fft_cols_tile_ok(c->N, t.inv_x) ? t.inv_x : 0;
-  c->tuning.fwd_x = c->tiles.fwd_x ? c->tiles.fwd_x : fft_cols_default_tile(c->N);
-  c->tuning.fwd_z = c->tiles.fwd_z ? c->tiles.fwd_z : fft_cols_default_tile(c->N);
-  c->tuning.inv_x = c->tiles.inv_x ? c->tiles.inv_x : fft_cols_default_tile(c->N);
-  c->plane_fwd = t.plane_fwd > 0 && spatial_plane_ok(c->N);
-  c->tuning.plane_fwd = c->plane_fwd ? 1 : -1;
-  c->tuning.nn_lanes = (t.nn_lanes == 1 || t.nn_lanes == 2 || t.nn_lanes == 4 ||
-                        t.nn_lanes == 8 || t.nn_lanes == 16)
-                           ? t.nn_lanes
-                           : 0;
-  c->tiles.fused_reg = t.fused_reg > 0 && spatial_reg(c->N);
-  c->tuning.fused_reg = c->tiles.fused_reg ? 1 : -1;
-  c->so3_reg = t.so3_reg > 0 && so3_reg_ok(c->Bo);
-  c->tuning.so3_reg = c->so3_reg ? 1 : -1;
-  c->occ_fwd = t.occ_fwd >= 0;
-  c->tuning.occ_fwd = c->occ_fwd ? 1 : -1;
-  c->inv_plane = t.inv_plane >= 0;
-  c->tuning.inv_plane = c->inv_plane ? 1 : -1;
-  c->nn_xcd = t.nn_xcd == 0 ? kNnXcdDefault : t.nn_xcd > 0;
-  c->tuning.nn_xcd = c->nn_xcd ? 1 : -1;
-  c->nn_seed = t.nn_seed == 0 ? kNnSeedDefault : (t.nn_seed > 0 ? (t.nn_seed & 3) : 0);
-  c->tuning.nn_seed = c->nn_seed ? c->nn_seed : -1;
-  c->xz_slab = t.xz_slab > 0;
-  c->tuning.xz_slab = c->xz_slab ? 1 : -1;
 }
 
 int phz_set_tuning(phz_ctx* c, const phz_tuning* t) {

@@ -94,3 +94,22 @@ def failed_launch(hip, kernel, call):
     ("k_spat_cross_z", "spatial")])
 def test_accumulators_are_cleared_after_a_failed_call(fake, kernel, call):
     _run(fake, "failed_launch", kernel, call)
+
+
+def zero_tuning(hip, B, N):
+    """phz_set_tuning with every field 0, or one set, leaves the others as a new
+    context has them; -1 is off."""
+    from phaser_amd.capi import Context
+    with Context(bandwidth=B, n_voxels=N, max_points=16) as ctx:
+        new = ctx.tuning()
+        ctx.set_tuning()
+        assert ctx.tuning() == new
+        ctx.set_tuning(nn_lanes=4)
+        assert ctx.tuning() == dict(new, nn_lanes=4)
+        ctx.set_tuning(fused_reg=-1, so3_reg=-1)
+        assert ctx.tuning() == dict(new, fused_reg=-1, so3_reg=-1)
+
+
+@pytest.mark.parametrize("B,N", [(64, 128), (50, 100), (31, 49), (8, 200)])
+def test_zero_tuning_fields_are_the_defaults(fake, B, N):
+    _run(fake, "zero_tuning", B, N)
