@@ -362,13 +362,15 @@ typedef struct {
   int32_t so3_reg;     /* the SO(3) alpha and gamma passes on the register kernels
                           (the engine's lengths, and n = 250, 288, 300, 320): 0 or
                           1 = on (default), -1 = off */
-  int32_t occ_fwd;     /* with fused_reg and the register engine for the forward
-                          z pass: that pass runs inside the cross-spectrum
-                          kernel (its output is never stored), and with the
-                          register engine for the x pass too, the r2c, x and z
-                          passes read and write only the voxel rows and z
-                          planes that hold points (the rest of the transform
-                          is zero): 0 or 1 = on (default), -1 = off */
+  int32_t occ_fwd;     /* the forward z pass inside the cross-spectrum kernel (its
+                          output is never stored), and the r2c, x and z passes
+                          over the voxel rows and z planes that hold points only
+                          (the rest of the transform is zero): 0 or 1 = on
+                          (default), -1 = off.  With fused_reg this needs fwd_z = 1,
+                          and the skipping fwd_x = 1 too; without it (off, or other
+                          lengths) fwd_x is the tile of the x pass and fwd_z that of
+                          the cross-spectrum kernel: 8, or else 16 up to N = 128.
+                          Not with plane_fwd or spatial zero padding */
   int32_t inv_plane;   /* with fused_reg and the register engine for the inverse x
                           pass (N <= 192): inverse x, c2r and argmax in one pass
                           over whole z planes in LDS: 0 or 1 = on (default), -1 = off */

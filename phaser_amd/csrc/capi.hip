@@ -841,7 +841,8 @@ int run_pairs(phz_ctx* c, int np, bool shared, hipStream_t s, float* d_rot_corr,
       if (occ) {
         if (!slab) reg->x_occ(2 * ncl, spec, occ_from(c), c->d_tw_N, s);
       } else if (lds_occ)
-        launch_spatial_fft_x_occ(N, 2 * ncl, spec, occ_from(c), c->plan_N, c->d_tw_N, s);
+        launch_spatial_fft_x_occ(N, 2 * ncl, spec, occ_from(c), c->tiles.fwd_x, c->plan_N, c->d_tw_N,
+                                 s);
       else if (!plane)
         launch_spatial_fft_pass(N, 2 * ncl, spec, 0, c->tiles.fwd_x, c->plan_N, c->d_tw_N, s);
       if (!zz && !lds_occ)
@@ -867,7 +868,7 @@ int run_pairs(phz_ctx* c, int np, bool shared, hipStream_t s, float* d_rot_corr,
       else if (lds_occ)
         launch_spatial_cross_zz(N, np, four ? F4 : Fc, fs, four ? G4 : Gc, gs, c->d_plane_occ,
                                 shared ? 0 : N, c->d_plane_occ + (int64_t)nt * N, N, c->vox.runs,
-                                c->plan_N, c->d_tw_N, c->d_work, s);
+                                c->tiles.fwd_z, c->plan_N, c->d_tw_N, c->d_work, s);
       else if (reg)
         reg->cross_z(np, four ? F4 : Fc, fs, four ? G4 : Gc, gs, c->vox.runs, true, c->d_tw_N,
                      c->d_work, s);

@@ -288,13 +288,16 @@ void launch_spatial_r2c(int N, int nclouds, const float* sumI, const float* sumR
                         const uint32_t* cnt, const FftPlan& plan, const float2* tw, float2* spec,
                         hipStream_t s, const uint8_t* row_occ = nullptr);
 // the same passes as SpatialReg's x_occ and cross_zz after an r2c with
-// row_occ (rows without points neither read nor written), any N <= 256
-void launch_spatial_fft_x_occ(int N, int nbatch, float2* spec, VoxelOcc occ, const FftPlan& plan,
-                              const float2* tw, hipStream_t s);
+// row_occ (rows without points neither read nor written), any N <= 256; it: the
+// columns per workgroup as in SpatialTiles (the register engine for the x pass
+// too), for the cross spectrum 8 or, up to N = 128, 16 (any other value)
+void launch_spatial_fft_x_occ(int N, int nbatch, float2* spec, VoxelOcc occ, int it,
+                              const FftPlan& plan, const float2* tw, hipStream_t s);
 void launch_spatial_cross_zz(int N, int npairs, ChannelSet F, int64_t f_stride, ChannelSet G,
                              int64_t g_stride, const uint8_t* f_occ, int64_t f_occ_stride,
                              const uint8_t* g_occ, int64_t g_occ_stride, const FusionRuns& runs,
-                             const FftPlan& plan, const float2* tw, float2* work, hipStream_t s);
+                             int it, const FftPlan& plan, const float2* tw, float2* work,
+                             hipStream_t s);
 void launch_spatial_fft_fwd(int N, int nspec, float2* spec, const FftPlan& plan,
                             const float2* tw, const SpatialTiles& tiles, hipStream_t s);
 // The passes of the translation stage on the register engine (fft_reg.hpp)

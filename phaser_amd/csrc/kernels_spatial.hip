@@ -1149,22 +1149,28 @@ void launch_spatial_r2c(int N, int nclouds, const float* sumI, const float* sumR
                      sumI, sumR, cnt, T, row_occ, plan, tw, spec, 2 * H, H);
 }
 
-void launch_spatial_fft_x_occ(int N, int nbatch, float2* spec, VoxelOcc occ, const FftPlan& plan,
-                              const float2* tw, hipStream_t s) {
+void launch_spatial_fft_x_occ(int N, int nbatch, float2* spec, VoxelOcc occ, int it,
+                              const FftPlan& plan, const float2* tw, hipStream_t s) {
   const int h = N / 2 + 1;
   const int64_t H = (int64_t)N * N * h;
-  if (N <= 128)
-    fft_cols_it<-1, 16>(spec, nbatch, H, N, N, h, plan, tw, s, occ);
-  else
-    fft_cols_it<-1, 8>(spec, nbatch, H, N, N, h, plan, tw, s, occ);
+  if (!fft_cols_tile_ok(N, it)) it = fft_cols_default_tile(N);
+  switch (it) {
+    case kRegisterEngine: spatial_reg(N)->x_occ(nbatch, spec, occ, tw, s); break;
+    case 8: fft_cols_it<-1, 8>(spec, nbatch, H, N, N, h, plan, tw, s, occ); break;
+    case 16: fft_cols_it<-1, 16>(spec, nbatch, H, N, N, h, plan, tw, s, occ); break;
+    case 32: fft_cols_it<-1, 32>(spec, nbatch, H, N, N, h, plan, tw, s, occ); break;
+    default: fft_cols_it<-1, 64>(spec, nbatch, H, N, N, h, plan, tw, s, occ); break;
+  }
 }
 
 void launch_spatial_cross_zz(int N, int npairs, ChannelSet F, int64_t f_stride, ChannelSet G,
                              int64_t g_stride, const uint8_t* f_occ, int64_t f_occ_stride,
                              const uint8_t* g_occ, int64_t g_occ_stride, const FusionRuns& runs,
-                             const FftPlan& plan, const float2* tw, float2* work, hipStream_t s) {
+                             int it, const FftPlan& plan, const float2* tw, float2* work,
+                             hipStream_t s) {
   const int inner = N * (N / 2 + 1);
-  if (N <= 128)
+  // the kernel holds 16 columns up to N = 128, 8 beyond
+  if (N <= 128 && it != 8)
     hipLaunchKernelGGL(k_spat_cross_zz<16>, dim3((inner + 15) / 16, npairs), dim3(256),
                        (4 * 16 * (N + 1) + N) * sizeof(float2), s, N, F, f_stride, G, g_stride,
                        f_occ, f_occ_stride, g_occ, g_occ_stride, runs, plan, tw, work);

@@ -72,6 +72,25 @@ def test_occupancy_skipping_matches_dense(N, channels):
             assert ra[k]["rot_index"] == rb[k]["rot_index"]
 
 
+@pytest.mark.parametrize("N,x,z", [(49, 8, 8), (49, 32, 16), (62, 64, 8), (127, 64, 16), (127, 8, 8),
+                                   (201, 16, 16), (100, 1, 8), (150, 1, 1), (200, 1, 8)])
+def test_occupancy_skipping_tiles(N, x, z):
+    """The tiles of the x pass and of the fused cross spectrum, and the register
+    engine's x pass between the LDS passes, against the dense passes."""
+    from phaser_amd.capi import Context
+    tgt, src = _cloud(9), _cloud(10, 2000)
+    with Context(bandwidth=8, n_voxels=N, max_points=6000) as ctx:
+        ctx.set_tuning(x, z, fused_reg=-1)
+        assert ctx.tuning()["fwd_x"] == x
+        a = ctx.register(tgt, src, grids=True)
+        ctx.set_tuning(8, 8, 8, fused_reg=-1, occ_fwd=-1)
+        b = ctx.register(tgt, src, grids=True)
+    err = _rel_any(a["trans_corr"], b["trans_corr"], N)
+    print(f"N {N}, tiles {x} {z}: {err:.2e}", flush=True)
+    assert err < 1e-5
+    assert a["trans_index"] == b["trans_index"]
+
+
 def _rel_any(a, b, N):
     if N % 2 == 0:
         return _rel_without_ties(a, b, N)[0]

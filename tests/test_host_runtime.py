@@ -58,10 +58,7 @@ def failed_launch(hip, kernel, call):
 
     with Context(bandwidth=8, n_voxels=8, max_points=64, max_batch=2, channels=4) as ctx:
         hip.reset()
-        try:
-            go(ctx)
-        except PhaserError as e:  # no kernel ran: the peak windows hold zeros
-            assert "error -4" in str(e), e
+        go(ctx)
         usual = hip.log()
         assert host_runtime.launches(usual, kernel), usual
         hip.reset()
@@ -76,10 +73,7 @@ def failed_launch(hip, kernel, call):
         fills = len(host_runtime.launches(usual, "k_fill_u32"))
         for cleared in (8, 0):  # the accumulators of four channels
             hip.reset()
-            try:
-                go(ctx)
-            except PhaserError as e:
-                assert "error -4" in str(e), e
+            go(ctx)
             log = hip.log()
             first = counts(log)[0]
             fill = host_runtime.launches(log, "k_fill_u32")
@@ -113,3 +107,29 @@ def zero_tuning(hip, B, N):
 @pytest.mark.parametrize("B,N", [(64, 128), (50, 100), (31, 49), (8, 200)])
 def test_zero_tuning_fields_are_the_defaults(fake, B, N):
     _run(fake, "zero_tuning", B, N)
+
+
+def tiles_of_a_call(hip, N, tile, fused):
+    """The tiles a caller sets are those of the kernels a call launches, in the
+    LDS passes that skip empty rows too (the cross spectrum's kernel has 8 and,
+    up to 128 voxels, 16 columns)."""
+    import numpy as np
+    from phaser_amd.capi import Context
+    cloud = np.ones((8, 4), np.float32)
+    with Context(bandwidth=8, n_voxels=N, max_points=16) as ctx:
+        ctx.set_tuning(fwd_x=tile, fwd_z=tile, fused_reg=fused)
+        assert ctx.tuning()["fwd_x"] == tile
+        hip.reset()
+        ctx.register(cloud, cloud)
+        log = hip.log()
+    x = [l for l in log if "k_fft_x_occ" in l or "k_fft_colsILin1" in l]
+    assert len(x) == 1
+    assert (f"k_fft_x_occILi{N}E" if tile == 1 else f"k_fft_colsILin1ELi{tile}E") in x[0], x
+    z = [l for l in log if "k_spat_cross" in l]
+    assert len(z) == 1 and f"k_spat_cross_zzILi{8 if tile == 8 or N > 128 else 16}E" in z[0], z
+
+
+@pytest.mark.parametrize("N,tile,fused", [(49, 8, 0), (49, 16, 0), (49, 32, 0), (127, 64, 0),
+                                          (201, 16, 0), (100, 1, -1), (100, 8, -1), (200, 1, -1)])
+def test_tiles_reach_the_kernels(fake, N, tile, fused):
+    _run(fake, "tiles_of_a_call", N, tile, fused)
