@@ -393,14 +393,18 @@ typedef struct {
                           other rounding): 1 = on, 0 or -1 = off (default: at
                           N = 128 it took 1.08 ms per 64 pairs against 0.85 ms
                           for the separate x pass and cross-spectrum kernel) */
-  float ms_fwd_x, ms_fwd_z, ms_inv_x;  /* per launch at max_batch (phz_autotune) */
-  float ms_plane;      /* plane pass per launch, or the r2c + x passes it replaces */
-  float ms_fused;      /* the three fused passes at max_batch, chosen form */
+  float ms_fwd_x, ms_fwd_z, ms_inv_x;  /* from phz_autotune: a column pass alone over
+                          every spectrum at max_batch with the chosen tile */
+  float ms_plane;      /* the translation stage's transforms at max_batch with the
+                          plane pass (0: not timed) */
+  float ms_fused;      /* the same in the chosen form */
   float ms_so3;        /* SO(3) alpha + gamma at max_batch, chosen form */
 } phz_tuning;
-/* Times every tile of each pass, and the plane pass against the r2c + x
- * passes it replaces, on the context's buffers at max_batch (repeats
- * launches each, after one warm-up round); keeps the fastest. */
+/* Times the translation stage's transforms at max_batch on a synthetic scan
+ * under other choices than a new context's (the LDS passes, the plane pass, the
+ * tiles of the passes that the form has; repeats runs each after a warm-up), and
+ * the SO(3) passes on both engines; keeps one that is more than 3% faster.
+ * The nn and xz_slab fields stay as they are. */
 int phz_autotune(phz_ctx* ctx, int repeats, phz_tuning* out);
 int phz_get_tuning(const phz_ctx* ctx, phz_tuning* out);
 int phz_set_tuning(phz_ctx* ctx, const phz_tuning* tuning);

@@ -687,94 +687,15 @@ ChannelSet channels(const float2* a, const float2* b, int C) {
   return cs;
 }
 
-// The registration pipeline on cloud slots [0, nt) targets and
-// [nt, nt+np) sources already resident in ctx->d_pts / d_npts.
-int run_pairs(phz_ctx* c, int np, bool shared, hipStream_t s, float* d_rot_corr,
-              float* d_trans_corr) {
-  // the peak-window fits read the grids: written to the context's own
-  // buffers when the caller wants none
-  const int kb = rot_neighbors(c->cfg), kg = pos_neighbors(c->cfg);
-  const bool bmm = c->cfg.rot_eval == PHZ_EVAL_MIXTURE, gmm = c->cfg.pos_eval == PHZ_EVAL_MIXTURE;
-  if (!d_rot_corr && kb > 0) d_rot_corr = c->d_peak_rot;
-  if (!d_trans_corr && kg > 0) d_trans_corr = c->d_peak_trans;
-  const int nt = shared ? 1 : np;
-  const int ncl = nt + np;
-  const int B = c->B, n = c->n, N = c->N;
-  const int64_t nq = (int64_t)n * n, BB = (int64_t)B * B;
-  // four channels: each cloud's reflectivity and ambient grids follow all
-  // clouds' range and intensity grids (and so do their coefficients)
+// The translation stage's transforms: the voxel accumulators of cloud slots
+// [0, nt) targets and [nt, nt+np) sources to the argmax partials of every
+// pair (their count per pair is returned) and, where given, its correlation
+// grid.  clear: zero the accumulators behind their last reader.
+int spatial_passes(phz_ctx* c, int np, bool shared, hipStream_t s, float* d_trans_corr,
+                   bool clear) {
+  const int nt = shared ? 1 : np, ncl = nt + np, N = c->N;
   const bool four = c->cfg.channels == 4;
-  // rotation
-  {
-    StageScope t(c, kS2Cells, s);
-    launch_s2_cells(c->d_pts, c->d_npts, c->cap, ncl, n, c->cells, s);
-  }
-  // SphRegistration: one sampled channel 0.6 intensity + 0.4 range per cloud
-  // (spherical-correlation.cc:103-112), transformed straight into the
-  // correlation's coefficients; no fusion, and reflectivity / ambient take
-  // no part in the rotation
-  const bool sph = c->cfg.method == PHZ_METHOD_SPH;
-  {
-    StageScope t(c, kS2NN, s);
-    launch_s2_nn(c->cap, ncl, n, c->d_grid, c->d_theta, c->max_sq, c->cells, c->d_grids,
-                 c->tuning.nn_lanes, s, four && !sph ? c->d_extra : nullptr,
-                 four && !sph ? c->d_grids + 2 * ncl * nq : nullptr, c->nn_xcd, sph,
-                 c->nn_seed);
-  }
-  {
-    StageScope t(c, kS2Transform, s);
-    if (sph)
-      launch_fst(c->d_grids, ncl, B, c->d_leg, c->d_leg_off, c->d_tw_n, c->d_F, c->d_fused,
-                 c->cfg.precision, s);
-    else
-      launch_fst(c->d_grids, (four ? 4 : 2) * ncl, B, c->d_leg, c->d_leg_off, c->d_tw_n, c->d_F,
-                 c->d_coef, c->cfg.precision, s);
-  }
-  if (!sph) {  // spherical order {range, intensity, refl, amb} (refl = amb = 0 with
-            // two channels), one launch for all clouds
-    StageScope t(c, kFuse, s);
-    ChannelSet cs = channels(c->d_coef, c->d_coef + BB, 4);
-    if (four) {
-      cs.ch[2] = c->d_coef + 2 * ncl * BB;
-      cs.ch[3] = c->d_coef + 2 * ncl * BB + BB;
-    }
-    launch_fuse(cs, (uint32_t)BB, c->s2.runs, c->d_fused, s, ncl, 2 * BB);
-    // spherical zero padding: the coefficients of degree < B in the layout of
-    // the correlation bandwidth Bo, zero above
-    if (c->Bo != B)
-      launch_pad_coef(c->d_fused, BB, c->d_pad_map, (int64_t)c->Bo * c->Bo, c->d_fused_o, ncl, s);
-  }
-  // the SO(3) correlation at Bo = B + spherical_zero_padding
-  const int Bo = c->Bo;
-  const int64_t BBo = (int64_t)Bo * Bo, no3 = (int64_t)c->no * c->no * c->no;
-  {
-    StageScope t(c, kSo3Synth, s);
-    launch_so3_synth(Bo, c->d_fused_o, shared ? 0 : BBo, c->d_fused_o + nt * BBo, BBo, np,
-                     c->d_wig, c->d_wig_off, c->d_wig_norm, c->d_S, c->cfg.precision, s,
-                     c->d_wig_hl, c->d_wig_hl_off);
-  }
-  {
-    StageScope t(c, kSo3Alpha, s);
-    launch_so3_fft_alpha(Bo, np, c->d_S, c->plan_no, c->d_tw_no, c->d_U, s, c->so3_reg);
-  }
-  int rot_partials = 0;
-  {
-    StageScope t(c, kSo3Gamma, s);
-    rot_partials = launch_so3_fft_gamma(Bo, np, c->d_U, c->plan_no, c->d_tw_no, d_rot_corr, no3,
-                                        c->d_partials, s, c->so3_reg);
-  }
-  {
-    StageScope t(c, kRotPose, s);
-    launch_rot_pose(Bo, np, c->d_partials, rot_partials, d_rot_corr, no3, kb, c->d_pose, s,
-                    c->cfg.skip_rot_axes, bmm);
-  }
-  // translation (accumulators are zero on entry and cleared again below)
   int trans_partials = 0;
-  {
-    StageScope t(c, kVoxelScatter, s);
-    launch_voxel_scatter(c->d_pts, c->d_npts, c->cap, ncl, c->d_pose, nt, N, c->d_edges, c->d_sumI,
-                         c->d_sumR, c->d_cnt, occ_from(c), s, extra_from(c));
-  }
   // spatial order {intensity, range, refl=0, amb=0}; pair p: target p (or
   // the shared target 0) against source nt+p
   const float2* F = c->d_spec;
@@ -878,7 +799,7 @@ int run_pairs(phz_ctx* c, int np, bool shared, hipStream_t s, float* d_rot_corr,
     }
     // after the last reader of the occupancy bytes (the cross spectrum
     // reads the plane bytes)
-    {
+    if (clear) {
       StageScope t(c, kVoxelClear, s);
       launch_voxel_clear(c->d_pts, c->d_npts, c->cap, ncl, c->d_pose, nt, N, c->d_edges, c->d_sumI,
                          c->d_sumR, c->d_cnt, occ_from(c), s, extra_from(c));
@@ -921,6 +842,97 @@ int run_pairs(phz_ctx* c, int np, bool shared, hipStream_t s, float* d_rot_corr,
       }
     }
   }
+  return trans_partials;
+}
+
+// The registration pipeline on cloud slots [0, nt) targets and
+// [nt, nt+np) sources already resident in ctx->d_pts / d_npts.
+int run_pairs(phz_ctx* c, int np, bool shared, hipStream_t s, float* d_rot_corr,
+              float* d_trans_corr) {
+  // the peak-window fits read the grids: written to the context's own
+  // buffers when the caller wants none
+  const int kb = rot_neighbors(c->cfg), kg = pos_neighbors(c->cfg);
+  const bool bmm = c->cfg.rot_eval == PHZ_EVAL_MIXTURE, gmm = c->cfg.pos_eval == PHZ_EVAL_MIXTURE;
+  if (!d_rot_corr && kb > 0) d_rot_corr = c->d_peak_rot;
+  if (!d_trans_corr && kg > 0) d_trans_corr = c->d_peak_trans;
+  const int nt = shared ? 1 : np;
+  const int ncl = nt + np;
+  const int B = c->B, n = c->n, N = c->N;
+  const int64_t nq = (int64_t)n * n, BB = (int64_t)B * B;
+  // four channels: each cloud's reflectivity and ambient grids follow all
+  // clouds' range and intensity grids (and so do their coefficients)
+  const bool four = c->cfg.channels == 4;
+  // rotation
+  {
+    StageScope t(c, kS2Cells, s);
+    launch_s2_cells(c->d_pts, c->d_npts, c->cap, ncl, n, c->cells, s);
+  }
+  // SphRegistration: one sampled channel 0.6 intensity + 0.4 range per cloud
+  // (spherical-correlation.cc:103-112), transformed straight into the
+  // correlation's coefficients; no fusion, and reflectivity / ambient take
+  // no part in the rotation
+  const bool sph = c->cfg.method == PHZ_METHOD_SPH;
+  {
+    StageScope t(c, kS2NN, s);
+    launch_s2_nn(c->cap, ncl, n, c->d_grid, c->d_theta, c->max_sq, c->cells, c->d_grids,
+                 c->tuning.nn_lanes, s, four && !sph ? c->d_extra : nullptr,
+                 four && !sph ? c->d_grids + 2 * ncl * nq : nullptr, c->nn_xcd, sph,
+                 c->nn_seed);
+  }
+  {
+    StageScope t(c, kS2Transform, s);
+    if (sph)
+      launch_fst(c->d_grids, ncl, B, c->d_leg, c->d_leg_off, c->d_tw_n, c->d_F, c->d_fused,
+                 c->cfg.precision, s);
+    else
+      launch_fst(c->d_grids, (four ? 4 : 2) * ncl, B, c->d_leg, c->d_leg_off, c->d_tw_n, c->d_F,
+                 c->d_coef, c->cfg.precision, s);
+  }
+  if (!sph) {  // spherical order {range, intensity, refl, amb} (refl = amb = 0 with
+            // two channels), one launch for all clouds
+    StageScope t(c, kFuse, s);
+    ChannelSet cs = channels(c->d_coef, c->d_coef + BB, 4);
+    if (four) {
+      cs.ch[2] = c->d_coef + 2 * ncl * BB;
+      cs.ch[3] = c->d_coef + 2 * ncl * BB + BB;
+    }
+    launch_fuse(cs, (uint32_t)BB, c->s2.runs, c->d_fused, s, ncl, 2 * BB);
+    // spherical zero padding: the coefficients of degree < B in the layout of
+    // the correlation bandwidth Bo, zero above
+    if (c->Bo != B)
+      launch_pad_coef(c->d_fused, BB, c->d_pad_map, (int64_t)c->Bo * c->Bo, c->d_fused_o, ncl, s);
+  }
+  // the SO(3) correlation at Bo = B + spherical_zero_padding
+  const int Bo = c->Bo;
+  const int64_t BBo = (int64_t)Bo * Bo, no3 = (int64_t)c->no * c->no * c->no;
+  {
+    StageScope t(c, kSo3Synth, s);
+    launch_so3_synth(Bo, c->d_fused_o, shared ? 0 : BBo, c->d_fused_o + nt * BBo, BBo, np,
+                     c->d_wig, c->d_wig_off, c->d_wig_norm, c->d_S, c->cfg.precision, s,
+                     c->d_wig_hl, c->d_wig_hl_off);
+  }
+  {
+    StageScope t(c, kSo3Alpha, s);
+    launch_so3_fft_alpha(Bo, np, c->d_S, c->plan_no, c->d_tw_no, c->d_U, s, c->so3_reg);
+  }
+  int rot_partials = 0;
+  {
+    StageScope t(c, kSo3Gamma, s);
+    rot_partials = launch_so3_fft_gamma(Bo, np, c->d_U, c->plan_no, c->d_tw_no, d_rot_corr, no3,
+                                        c->d_partials, s, c->so3_reg);
+  }
+  {
+    StageScope t(c, kRotPose, s);
+    launch_rot_pose(Bo, np, c->d_partials, rot_partials, d_rot_corr, no3, kb, c->d_pose, s,
+                    c->cfg.skip_rot_axes, bmm);
+  }
+  // translation (accumulators are zero on entry and cleared again below)
+  {
+    StageScope t(c, kVoxelScatter, s);
+    launch_voxel_scatter(c->d_pts, c->d_npts, c->cap, ncl, c->d_pose, nt, N, c->d_edges, c->d_sumI,
+                         c->d_sumR, c->d_cnt, occ_from(c), s, extra_from(c));
+  }
+  const int trans_partials = spatial_passes(c, np, shared, s, d_trans_corr, true);
   {
     StageScope t(c, kTransPose, s);
     // with padding the window and the metres use Np voxels and the
@@ -1852,148 +1864,163 @@ int phz_get_tuning(const phz_ctx* c, phz_tuning* t) {
   return 0;
 }
 
+// The whole translation stage under candidate choices, on a synthetic scan in
+// every cloud slot, as a call at max_batch runs it: an option that suits one
+// pass can cost more in the others (an LDS tile or the plane pass switches the
+// skipping of empty rows and planes off).  A new context's choices stay unless
+// another one is faster by more than two timings of one form differ.
 int phz_autotune(phz_ctx* c, int repeats, phz_tuning* out) {
   PHZ_CHECK(c, "null argument");
   PHZ_CHECK(repeats >= 1 && repeats <= 1000, "repeats out of range");
+  constexpr float kMargin = 0.97f;
   hipStream_t s = c->stream;
-  const int N = c->N, P = c->cfg.max_batch, nspec = 2 * c->max_clouds;
-  // timing runs on the context's own spectra buffers at full batch size
-  launch_fill_u32((uint32_t*)c->d_spec, (size_t)2 * nspec * c->H, 0u, s);
-  launch_fill_u32((uint32_t*)c->d_work, (size_t)2 * P * c->H, 0u, s);
-  hipEvent_t a, b;
-  PHZ_HIP(hipEventCreate(&a));
-  PHZ_HIP(hipEventCreate(&b));
-  const int cands[5] = {kRegisterEngine, 8, 16, 32, 64};
-  phz_tuning best{};
-  float best_ms[3] = {1e30f, 1e30f, 1e30f};
+  const int N = c->N, P = c->cfg.max_batch, M = c->max_clouds;
+  const bool padded = c->sp > 0;
+  const phz_tuning before = c->tuning;
+  const bool profiling = c->profiling;
   int rc = 0;
-  for (int site = 0; site < 3 && !rc; ++site)
-    for (int it : cands) {
-      if (!fft_cols_tile_ok(N, it)) continue;
-      float ms = 0.f;
-      for (int pass = 0; pass < 2; ++pass) {  // pass 0 warms up
-        if (hipEventRecord(a, s) != hipSuccess) rc = -2;
-        for (int r = 0; r < repeats; ++r)
-          launch_spatial_fft_pass(N, site == 2 ? P : nspec, site == 2 ? c->d_work : c->d_spec,
-                                  site, it, c->plan_N, c->d_tw_N, s);
-        if (hipEventRecord(b, s) != hipSuccess || hipEventSynchronize(b) != hipSuccess ||
-            hipEventElapsedTime(&ms, a, b) != hipSuccess)
-          rc = -2;
-      }
-      ms /= (float)repeats;
-      if (ms < best_ms[site]) {
-        best_ms[site] = ms;
-        (site == 0 ? best.fwd_x : site == 1 ? best.fwd_z : best.inv_x) = it;
-      }
+  hipEvent_t a = nullptr, b = nullptr;
+  // ms of one run of f; the first one is not timed, and one slower than limit
+  // is not repeated
+  auto timed = [&](auto f, float limit) {
+    float ms = 0.f;
+    f();
+    for (int pass = 0; pass < 2 && !rc; ++pass) {
+      if (hipEventRecord(a, s) != hipSuccess) rc = -2;
+      for (int r = 0; r < (pass ? repeats : 1); ++r) f();
+      if (hipEventRecord(b, s) != hipSuccess || hipEventSynchronize(b) != hipSuccess ||
+          hipEventElapsedTime(&ms, a, b) != hipSuccess || hipGetLastError() != hipSuccess)
+        rc = -2;
+      if (pass == 0 && ms > limit) return ms;
     }
-  // the plane pass against the r2c + x passes it replaces (best x tile)
-  float plane_ms = 0.f, classic_ms = 0.f;
-  if (!rc && spatial_plane_ok(N)) {
-    const int ncl = c->max_clouds;
-    for (int variant = 0; variant < 2 && !rc; ++variant) {
-      float ms = 0.f;
-      for (int pass = 0; pass < 2; ++pass) {
-        if (hipEventRecord(a, s) != hipSuccess) rc = -2;
-        for (int r = 0; r < repeats; ++r) {
-          if (variant == 0) {
-            launch_spatial_plane_fwd(N, ncl, c->d_sumI, c->d_sumR, c->d_cnt, c->plan_N,
-                                     c->d_tw_N, c->d_spec, s);
-          } else {
-            launch_spatial_r2c(N, ncl, c->d_sumI, c->d_sumR, c->d_cnt, c->plan_N, c->d_tw_N,
-                               c->d_spec, s);
-            launch_spatial_fft_pass(N, nspec, c->d_spec, 0, best.fwd_x, c->plan_N, c->d_tw_N, s);
-          }
-        }
-        if (hipEventRecord(b, s) != hipSuccess || hipEventSynchronize(b) != hipSuccess ||
-            hipEventElapsedTime(&ms, a, b) != hipSuccess)
-          rc = -2;
-      }
-      (variant == 0 ? plane_ms : classic_ms) = ms / (float)repeats;
+    return ms / (float)repeats;
+  };
+  AccumulatorUse use(c, s);
+  TRY(use.begin());
+  {
+    // 64 rings of a scanner in the middle of the grid: ground below, walls
+    // around at 0.3 to 0.6 of its half width
+    const int n = (int)std::min<int64_t>(c->cap, 65536), ring = std::max(n / 64, 1);
+    std::vector<float> scan((size_t)n * 4);
+    const float mid = 0.5f * (c->vox.lo + c->vox.hi), half = 0.5f * (c->vox.hi - c->vox.lo);
+    for (int i = 0; i < n; ++i) {
+      const float az = 6.2831853f * (float)(i % ring) / (float)ring;
+      const float el = -0.44f + 0.7f * (float)(i / ring % 64) / 64.f;
+      const float wall = half * (0.45f + 0.15f * std::sin(3.f * az)), low = -0.04f * half;
+      const float dist = el < 0.f ? std::min(wall, low / std::tan(el)) : wall;
+      scan[4 * i] = mid + dist * std::cos(az);
+      scan[4 * i + 1] = mid + dist * std::sin(az);
+      scan[4 * i + 2] = mid + dist * std::tan(el);
+      scan[4 * i + 3] = (float)(1 + i % 97);
     }
-    best.plane_fwd = plane_ms <= classic_ms ? 1 : -1;
-  } else {
-    best.plane_fwd = -1;
+    for (int k = 0; k < M; ++k)
+      TRY(load_cloud(c, k, k ? (const float*)c->d_pts : scan.data(), n,
+                     k ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
+    TRY(commit_counts(c, M, s));
+    launch_voxel_scatter(c->d_pts, c->d_npts, c->cap, M, nullptr, 0, N, c->d_edges, c->d_sumI,
+                         c->d_sumR, c->d_cnt, occ_from(c), s, extra_from(c));
+    PHZ_HIP(hipGetLastError());
+    PHZ_HIP(hipStreamSynchronize(s));
   }
-  // the fused passes (r2c, cross_z, c2r): register engine against LDS kernels
-  float fused_ms[2] = {0.f, 0.f};
-  if (const SpatialReg* reg = spatial_reg(N); !rc && reg) {
-    const int ncl = c->max_clouds;
-    const float2* F = c->d_spec;
-    const float2* G = c->d_spec + (int64_t)2 * c->H;
-    for (int variant = 0; variant < 2 && !rc; ++variant) {
-      float ms = 0.f;
-      for (int pass = 0; pass < 2; ++pass) {
-        if (hipEventRecord(a, s) != hipSuccess) rc = -2;
-        for (int r = 0; r < repeats; ++r) {
-          if (variant == 1) {
-            reg->r2c(ncl, c->d_sumI, c->d_sumR, c->d_cnt, nullptr, false, c->d_tw_N, c->d_spec, s);
-            reg->cross_z(P, channels(F, F + c->H, 4), 0, channels(G, G + c->H, 4), 0, c->vox.runs,
-                         true, c->d_tw_N, c->d_work, s);
-            reg->c2r(P, c->d_work, c->d_tw_N, nullptr, c->d_partials, s);
-          } else {
-            launch_spatial_r2c(N, ncl, c->d_sumI, c->d_sumR, c->d_cnt, c->plan_N, c->d_tw_N,
-                               c->d_spec, s);
-            launch_spatial_cross_z(N, P, channels(F, F + c->H, 4), 0, channels(G, G + c->H, 4), 0,
-                                   c->vox.runs, true, c->plan_N, c->d_tw_N, c->d_work, s);
-            launch_spatial_c2r(N, P, c->d_work, c->plan_N, c->d_tw_N, nullptr, c->d_partials,
-                               c->d_keys, s);
-          }
-        }
-        if (hipEventRecord(b, s) != hipSuccess || hipEventSynchronize(b) != hipSuccess ||
-            hipEventElapsedTime(&ms, a, b) != hipSuccess)
-          rc = -2;
-      }
-      fused_ms[variant] = ms / (float)repeats;
+  if (hipEventCreate(&a) != hipSuccess || hipEventCreate(&b) != hipSuccess) rc = -2;
+  c->profiling = false;
+  phz_tuning best{}, t{};
+  best.nn_lanes = before.nn_lanes;  // data-dependent: set with phz_set_tuning
+  best.nn_xcd = before.nn_xcd;
+  best.nn_seed = before.nn_seed;
+  best.xz_slab = before.xz_slab;
+  float best_ms = 1e30f, plane_ms = 0.f;
+  auto consider = [&](const phz_tuning& next) {
+    if (rc) return 0.f;
+    apply_tuning(c, next);
+    const float ms = timed([&] { spatial_passes(c, P, false, s, c->d_peak_trans, false); },
+                           1.5f * best_ms);
+    if (!rc && ms < kMargin * best_ms) {
+      best = c->tuning;
+      best_ms = ms;
     }
-    best.fused_reg = fused_ms[1] <= fused_ms[0] ? 1 : -1;
-  } else {
-    best.fused_reg = -1;
+    return ms;
+  };
+  // the tiles of a site but for the one in use, up to a number of columns
+  auto tiles = [&](int32_t phz_tuning::*site, int most = 64) {
+    const int now = best.*site;
+    for (int it : {kRegisterEngine, 8, 16, 32, 64}) {
+      if (it == now || it > most || !fft_cols_tile_ok(N, it)) continue;
+      t = best;
+      t.*site = it;
+      consider(t);
+    }
+  };
+  consider(best);
+  if (spatial_reg(N)) {
+    t = best;
+    t.fused_reg = -1;
+    consider(t);
   }
+  if (spatial_plane_ok(N) && c->cfg.channels != 4) {
+    t = best;
+    t.plane_fwd = 1;
+    plane_ms = consider(t);
+  }
+  // the tiles where the chosen form has such a pass: the register engine's
+  // forward passes are not tiled unless the grid is padded
+  const bool reg = best.fused_reg > 0;
+  if (!reg || padded) {
+    if (best.plane_fwd < 0) tiles(&phz_tuning::fwd_x);
+    // a z pass of its own, or the fused cross spectrum's 8 or 16 columns
+    if (padded || best.plane_fwd > 0) tiles(&phz_tuning::fwd_z);
+    else if (N <= 128) tiles(&phz_tuning::fwd_z, 8);
+  }
+  if (!padded && !(reg && spatial_reg(N)->inv_plane)) tiles(&phz_tuning::inv_x);
   // SO(3) alpha + gamma passes: register engine against LDS kernels
-  float so3_ms[2] = {0.f, 0.f};
-  if (!rc && so3_reg_ok(c->Bo)) {
-    const int B = c->Bo, n = c->no;
-    launch_fill_u32((uint32_t*)c->d_S, (size_t)2 * P * B * (2 * B - 1) * n, 0u, s);
-    for (int variant = 0; variant < 2 && !rc; ++variant) {
-      float ms = 0.f;
-      for (int pass = 0; pass < 2; ++pass) {
-        if (hipEventRecord(a, s) != hipSuccess) rc = -2;
-        for (int r = 0; r < repeats; ++r) {
-          launch_so3_fft_alpha(B, P, c->d_S, c->plan_no, c->d_tw_no, c->d_U, s, variant == 1);
-          launch_so3_fft_gamma(B, P, c->d_U, c->plan_no, c->d_tw_no, nullptr, (int64_t)n * n * n,
-                               c->d_partials, s, variant == 1);
-        }
-        if (hipEventRecord(b, s) != hipSuccess || hipEventSynchronize(b) != hipSuccess ||
-            hipEventElapsedTime(&ms, a, b) != hipSuccess)
-          rc = -2;
-      }
-      so3_ms[variant] = ms / (float)repeats;
-    }
-    best.so3_reg = so3_ms[1] <= so3_ms[0] ? 1 : -1;
-  } else {
-    best.so3_reg = -1;
+  float so3_ms = 0.f;
+  const int B = c->Bo, n = c->no;
+  launch_fill_u32((uint32_t*)c->d_S, (size_t)2 * P * B * (2 * B - 1) * n, 0u, s);
+  auto so3 = [&](bool engine, float limit) {
+    return timed([&] {
+      launch_so3_fft_alpha(B, P, c->d_S, c->plan_no, c->d_tw_no, c->d_U, s, engine);
+      launch_so3_fft_gamma(B, P, c->d_U, c->plan_no, c->d_tw_no, nullptr, (int64_t)n * n * n,
+                           c->d_partials, s, engine);
+    }, limit);
+  };
+  if (!rc) so3_ms = so3(so3_reg_ok(B), 1e30f);
+  if (!rc && so3_reg_ok(B)) {
+    const float lds_ms = so3(false, 1.5f * so3_ms);
+    best.so3_reg = lds_ms < kMargin * so3_ms ? -1 : 1;
+    so3_ms = std::min(so3_ms, lds_ms);
   }
-  (void)hipEventDestroy(a);
-  (void)hipEventDestroy(b);
+  // the column passes alone over every spectrum
+  float pass_ms[3] = {0.f, 0.f, 0.f};
+  launch_fill_u32((uint32_t*)c->d_spec, (size_t)4 * M * c->H, 0u, s);
+  launch_fill_u32((uint32_t*)c->d_work, (size_t)2 * P * c->H, 0u, s);
+  for (int site = 0; site < 3 && !rc; ++site) {
+    const int it = site == 0 ? best.fwd_x : site == 1 ? best.fwd_z : best.inv_x;
+    pass_ms[site] = timed([&] {
+      launch_spatial_fft_pass(N, site == 2 ? P : 2 * M, site == 2 ? c->d_work : c->d_spec, site,
+                              it, c->plan_N, c->d_tw_N, s);
+    }, 1e30f);
+  }
+  launch_voxel_clear(c->d_pts, c->d_npts, c->cap, M, nullptr, 0, N, c->d_edges, c->d_sumI,
+                     c->d_sumR, c->d_cnt, occ_from(c), s, extra_from(c));
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(s) != hipSuccess) rc = -2;
+  if (a) (void)hipEventDestroy(a);
+  if (b) (void)hipEventDestroy(b);
+  c->profiling = profiling;
+  clear_graphs(c);
   if (rc) {
+    apply_tuning(c, before);
+    c->tuning = before;
     set_error("autotune timing failed");
     return rc;
   }
-  best.nn_lanes = c->tuning.nn_lanes;  // data-dependent: set with phz_set_tuning
-  best.nn_xcd = c->tuning.nn_xcd;
-  best.nn_seed = c->tuning.nn_seed;
-  best.xz_slab = c->tuning.xz_slab;
-  best.ms_fwd_x = best_ms[0];
-  best.ms_fwd_z = best_ms[1];
-  best.ms_inv_x = best_ms[2];
+  use.end();
   apply_tuning(c, best);
-  clear_graphs(c);
-  c->tuning.ms_fwd_x = best_ms[0];
-  c->tuning.ms_fwd_z = best_ms[1];
-  c->tuning.ms_inv_x = best_ms[2];
-  c->tuning.ms_plane = best.plane_fwd > 0 ? plane_ms : classic_ms;
-  c->tuning.ms_fused = best.fused_reg > 0 ? fused_ms[1] : fused_ms[0];
-  c->tuning.ms_so3 = best.so3_reg > 0 ? so3_ms[1] : so3_ms[0];
+  c->tuning.ms_fwd_x = pass_ms[0];
+  c->tuning.ms_fwd_z = pass_ms[1];
+  c->tuning.ms_inv_x = pass_ms[2];
+  c->tuning.ms_plane = plane_ms;
+  c->tuning.ms_fused = best_ms;
+  c->tuning.ms_so3 = so3_ms;
   if (out) *out = c->tuning;
   return 0;
 }

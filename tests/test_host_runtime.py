@@ -133,3 +133,80 @@ def tiles_of_a_call(hip, N, tile, fused):
                                           (201, 16, 0), (100, 1, -1), (100, 8, -1), (200, 1, -1)])
 def test_tiles_reach_the_kernels(fake, N, tile, fused):
     _run(fake, "tiles_of_a_call", N, tile, fused)
+
+
+def tuned(hip, N, pad, costs, want, kernels):
+    """phz_autotune under kernels of given costs, from a new context: the fields
+    it changes, and the kernels that the next call then launches."""
+    import numpy as np
+    from phaser_amd.capi import Context
+    cloud = np.ones((8, 4), np.float32)
+    with Context(bandwidth=8, n_voxels=N, max_points=16, max_batch=3,
+                 spatial_zero_padding=pad) as ctx:
+        new = ctx.tuning()
+        hip.reset()
+        for kernel, ms in costs.items():
+            hip.cost(kernel, ms)
+        t = ctx.autotune(repeats=2)
+        timed = {k for k in t if k.startswith("ms_")}
+        assert {k: t[k] for k in t if k not in timed and t[k] != new[k]} == want
+        assert t["ms_fused"] > 0 and t["ms_fwd_x"] > 0
+        ctx.register(cloud, cloud)
+        hip.reset()
+        ctx.register(cloud, cloud)
+        log = hip.log()
+        assert len(host_runtime.launches(log, "k_fill_u32")) == 0
+        for k in kernels:
+            assert host_runtime.launches(log, k), (k, log)
+
+
+@pytest.mark.parametrize("N,pad,costs,want,kernels", [
+    # the plane pass beats the dense LDS passes, and not those of a call
+    (100, 0, {"k_spat_plane_fwd": 5.0, "k_spat_r2cI": 9.0, "k_spat_r2c_rows": 0.5}, {},
+     ["k_spat_r2c_rows", "k_fft_x_occ"]),
+    # so does an LDS tile of a pass that a call does not run alone
+    (100, 0, {"k_fft_lines": 9.0, "k_spat_cross_z_reg": 5.0, "k_spat_plane_fwd": 5.0}, {},
+     ["k_spat_cross_zz_reg"]),
+    # nothing differs by more than the margin
+    (128, 0, {"k_spat": 1.0, "k_fft": 1.0, "k_spat_r2c_rows": 0.02, "k_fft_x_occ": 0.02,
+                  "k_spat_plane_fwd": 0.95}, {},
+     ["k_spat_r2c_rows", "k_spat_inv_plane"]),
+    # whole forms that win
+    (100, 0, {"k_spat_r2c_rows": 50.0, "k_spat_plane_fwd": 90.0}, {"fused_reg": -1},
+     ["k_spat_r2cILb0E", "k_fft_x_occ", "k_spat_cross_zzI"]),
+    (49, 0, {"k_spat_r2cI": 5.0, "k_fft_colsILin1E": 5.0}, {"plane_fwd": 1}, ["k_spat_plane_fwd"]),
+    # tiles of the passes that a call runs
+    (49, 0, {"k_spat_plane_fwd": 90.0, "k_fft_colsILin1ELi16E": 4.0, "k_fft_colsILin1ELi8E": 3.0,
+             "k_spat_cross_zzILi16E": 2.0, "k_fft_colsILi1ELi16E": 2.0},
+     {"fwd_x": 32, "fwd_z": 8, "inv_x": 8},
+     ["k_fft_colsILin1ELi32E", "k_spat_cross_zzILi8E", "k_fft_colsILi1ELi8E"]),
+    (200, 0, {"k_fft_linesILi1E": 2.0, "k_fft_colsILi1ELi16E": 1.0}, {"inv_x": 8},
+     ["k_fft_colsILi1ELi8E", "k_spat_cross_zz_reg"]),
+    (62, 3, {"k_fft_colsILin1ELi16E": 4.0, "k_spat_plane_fwd": 90.0}, {"fwd_x": 8, "fwd_z": 8},
+     ["k_fft_colsILin1ELi8E", "k_spat_pad_gather"]),
+])
+def test_autotune_times_what_a_call_runs(fake, N, pad, costs, want, kernels):
+    _run(fake, "tuned", N, pad, costs, want, kernels)
+
+
+def failed_tuning(hip):
+    """A launch that fails leaves the choices as they were and an error, and
+    the next call clears the synthetic scan's voxels."""
+    import numpy as np
+    from phaser_amd.capi import Context, PhaserError
+    cloud = np.ones((8, 4), np.float32)
+    with Context(bandwidth=8, n_voxels=49, max_points=16) as ctx:
+        ctx.set_tuning(fwd_x=32, nn_lanes=2)
+        before = ctx.tuning()
+        hip.reset()
+        hip.fail("k_spat_cross_zz")
+        with pytest.raises(PhaserError, match="autotune"):
+            ctx.autotune(repeats=2)
+        assert ctx.tuning() == before
+        hip.reset()
+        ctx.register(cloud, cloud)
+        assert len(host_runtime.launches(hip.log(), "k_fill_u32")) == 6
+
+
+def test_failed_autotune(fake):
+    _run(fake, "failed_tuning")
