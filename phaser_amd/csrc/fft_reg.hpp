@@ -1,5 +1,6 @@
-// fft_reg.hpp -- register-resident FFTs of lengths 48..320 with factors 2, 3
-// and 5 for gfx950: each line is split as L = R1 * R2 (four-step Cooley-Tukey,
+// fft_reg.hpp -- register-resident FFTs of the lengths of PHZ_REG_LENGTHS (48 to
+// 256, even, with factors 2, 3 and 5) and, for the SO(3) grid, up to 320 for
+// gfx950: each line is split as L = R1 * R2 (four-step Cooley-Tukey,
 // n = n2 + R2 n1, k = k1 + R1 k2):
 //   X[k1 + R1 k2] = sum_n2 W_R2^(n2 k2) W_L^(n2 k1) sum_n1 x[n2 + R2 n1] W_R1^(n1 k1)
 // R2 threads per line each load R1 elements straight from HBM, transform
@@ -188,18 +189,25 @@ __host__ __device__ __forceinline__ void dft_reg(float2 (&v)[R]) {
   }
 }
 
-// The lengths of the engine and their splits.  R1 elements per thread and
-// R2 threads per line; a workgroup of LINES lines is whole waves.  R1 a multiple of R2, or R1 <= R2 near it: the second transforms
-// then take whole rounds or a single one (a partly filled second round, as
-// 12 x 10 for 120, made the fused cross spectrum twice as slow as one of
-// 10 x 12).  LINES = 32 lines make a strided pass read 256-byte runs; 16
+// The lengths of the engine and their splits; other lengths take the LDS
+// passes.  R1 elements per thread and R2 threads per line; a workgroup of LINES
+// lines is whole waves.  R1 a multiple of R2, or R1 <= R2 near it: the second
+// transforms then take whole rounds or a single one (a partly filled second
+// round, as 12 x 10 for 120, made the fused cross spectrum twice as slow as one
+// of 10 x 12).  LINES = 32 lines make a strided pass read 256-byte runs; 16
 // where 32 lines would need many more threads or span more than two z planes,
 // 64 for whole waves at odd R2.
-#define PHZ_REG_LENGTHS(X)                                                                     \
-  X(48, 12, 4) X(60, 5, 12) X(64, 8, 8) X(72, 12, 6) X(80, 8, 10) X(90, 9, 10) X(96, 8, 12)    \
-  X(100, 10, 10) X(108, 9, 12) X(120, 10, 12) X(128, 16, 8) X(144, 9, 16) X(150, 10, 15)       \
-  X(160, 10, 16) X(180, 10, 18) X(192, 12, 16) X(200, 20, 10) X(216, 12, 18) X(240, 15, 16)    \
-  X(256, 16, 16)
+// In groups, one per file that builds them for the translation stage.
+#define PHZ_REG_LENGTHS_A(X) \
+  X(48, 12, 4) X(60, 5, 12) X(64, 8, 8) X(72, 12, 6) X(80, 8, 10) X(90, 9, 10)
+#define PHZ_REG_LENGTHS_B(X) \
+  X(96, 8, 12) X(100, 10, 10) X(108, 9, 12) X(120, 10, 12) X(128, 16, 8)
+#define PHZ_REG_LENGTHS_C(X) X(144, 9, 16) X(150, 10, 15) X(160, 10, 16) X(180, 10, 18)
+#define PHZ_REG_LENGTHS_D(X) X(192, 12, 16) X(200, 20, 10) X(216, 12, 18)
+#define PHZ_REG_LENGTHS_E(X) X(240, 15, 16) X(256, 16, 16)
+#define PHZ_REG_LENGTHS(X)                                                          \
+  PHZ_REG_LENGTHS_A(X) PHZ_REG_LENGTHS_B(X) PHZ_REG_LENGTHS_C(X) PHZ_REG_LENGTHS_D(X) \
+  PHZ_REG_LENGTHS_E(X)
 // the SO(3) grid's sides 2 B reach 320
 #define PHZ_REG_LENGTHS_SO3(X) \
   PHZ_REG_LENGTHS(X) X(250, 25, 10) X(288, 16, 18) X(300, 15, 20) X(320, 16, 20)

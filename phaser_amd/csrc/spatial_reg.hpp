@@ -766,4 +766,14 @@ struct SpatialRegT {
 
 }  // namespace
 
+// NAME(N): the passes of length N, or null, for the lengths of LIST
+#define PHZ_SPATIAL_REG_OPS(LEN, A, B) SpatialRegT<LEN>::ops(),
+#define PHZ_SPATIAL_REG_GROUP(NAME, LIST)                         \
+  const SpatialReg* NAME(int N) {                                 \
+    static constexpr SpatialReg ops[] = {LIST(PHZ_SPATIAL_REG_OPS)}; \
+    for (const SpatialReg& o : ops)                               \
+      if (o.N == N) return &o;                                    \
+    return nullptr;                                               \
+  }
+
 }  // namespace phz

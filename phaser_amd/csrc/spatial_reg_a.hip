@@ -1,20 +1,6 @@
-// Register-engine passes of the translation stage for N = 48, 60, 64, 72, 80, 90.
+// Register-engine passes of the translation stage for the lengths of one group.
 #include "spatial_reg.hpp"
 
 namespace phz {
-
-const SpatialReg* spatial_reg_a(int N) {
-  static constexpr SpatialReg ops[] = {
-      SpatialRegT<48>::ops(),
-      SpatialRegT<60>::ops(),
-      SpatialRegT<64>::ops(),
-      SpatialRegT<72>::ops(),
-      SpatialRegT<80>::ops(),
-      SpatialRegT<90>::ops(),
-  };
-  for (const SpatialReg& o : ops)
-    if (o.N == N) return &o;
-  return nullptr;
-}
-
+PHZ_SPATIAL_REG_GROUP(spatial_reg_a, PHZ_REG_LENGTHS_A)
 }  // namespace phz

@@ -1,19 +1,6 @@
-// Register-engine passes of the translation stage for N = 96, 100, 108, 120, 128.
+// Register-engine passes of the translation stage for the lengths of one group.
 #include "spatial_reg.hpp"
 
 namespace phz {
-
-const SpatialReg* spatial_reg_b(int N) {
-  static constexpr SpatialReg ops[] = {
-      SpatialRegT<96>::ops(),
-      SpatialRegT<100>::ops(),
-      SpatialRegT<108>::ops(),
-      SpatialRegT<120>::ops(),
-      SpatialRegT<128>::ops(),
-  };
-  for (const SpatialReg& o : ops)
-    if (o.N == N) return &o;
-  return nullptr;
-}
-
+PHZ_SPATIAL_REG_GROUP(spatial_reg_b, PHZ_REG_LENGTHS_B)
 }  // namespace phz

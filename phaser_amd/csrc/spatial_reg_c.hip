@@ -1,18 +1,6 @@
-// Register-engine passes of the translation stage for N = 144, 150, 160, 180.
+// Register-engine passes of the translation stage for the lengths of one group.
 #include "spatial_reg.hpp"
 
 namespace phz {
-
-const SpatialReg* spatial_reg_c(int N) {
-  static constexpr SpatialReg ops[] = {
-      SpatialRegT<144>::ops(),
-      SpatialRegT<150>::ops(),
-      SpatialRegT<160>::ops(),
-      SpatialRegT<180>::ops(),
-  };
-  for (const SpatialReg& o : ops)
-    if (o.N == N) return &o;
-  return nullptr;
-}
-
+PHZ_SPATIAL_REG_GROUP(spatial_reg_c, PHZ_REG_LENGTHS_C)
 }  // namespace phz

@@ -1,17 +1,6 @@
-// Register-engine passes of the translation stage for N = 192, 200, 216.
+// Register-engine passes of the translation stage for the lengths of one group.
 #include "spatial_reg.hpp"
 
 namespace phz {
-
-const SpatialReg* spatial_reg_d(int N) {
-  static constexpr SpatialReg ops[] = {
-      SpatialRegT<192>::ops(),
-      SpatialRegT<200>::ops(),
-      SpatialRegT<216>::ops(),
-  };
-  for (const SpatialReg& o : ops)
-    if (o.N == N) return &o;
-  return nullptr;
-}
-
+PHZ_SPATIAL_REG_GROUP(spatial_reg_d, PHZ_REG_LENGTHS_D)
 }  // namespace phz

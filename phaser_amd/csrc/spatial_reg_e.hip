@@ -1,16 +1,6 @@
-// Register-engine passes of the translation stage for N = 240, 256.
+// Register-engine passes of the translation stage for the lengths of one group.
 #include "spatial_reg.hpp"
 
 namespace phz {
-
-const SpatialReg* spatial_reg_e(int N) {
-  static constexpr SpatialReg ops[] = {
-      SpatialRegT<240>::ops(),
-      SpatialRegT<256>::ops(),
-  };
-  for (const SpatialReg& o : ops)
-    if (o.N == N) return &o;
-  return nullptr;
-}
-
+PHZ_SPATIAL_REG_GROUP(spatial_reg_e, PHZ_REG_LENGTHS_E)
 }  // namespace phz
