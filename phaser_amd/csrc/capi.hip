@@ -344,7 +344,7 @@ size_t context_bytes(const phz_config& cf) {
   add(P * Bo * (2 * Bo - 1) * no, sizeof(float2));
   add(P * no * Bo * no, sizeof(float2));
   add(no * no * no, sizeof(float));
-  add(2 * P, sizeof(unsigned long long));
+  add(P, sizeof(unsigned long long));
   add(P * ppp, sizeof(unsigned long long));
   add(P, sizeof(DevPose));
   // voxel accumulators, spectra and the translation grid
@@ -625,7 +625,7 @@ int init_ctx(phz_ctx* c) {
   TRY(dalloc(c, &c->d_S, (size_t)P * Bo * (2 * Bo - 1) * no));
   TRY(dalloc(c, &c->d_U, (size_t)P * no * Bo * no));
   TRY(dalloc(c, &c->d_corr_rot, (size_t)no * no * no));
-  TRY(dalloc(c, &c->d_keys, (size_t)2 * P));
+  TRY(dalloc(c, &c->d_keys, (size_t)P));
   c->partials_per_pair = std::max(so3_gamma_blocks(c->Bo), spatial_c2r_blocks(c->Np));
   TRY(dalloc(c, &c->d_partials, (size_t)P * c->partials_per_pair));
   TRY(dalloc(c, &c->d_pose, (size_t)P));
@@ -742,10 +742,9 @@ int spatial_passes(phz_ctx* c, int np, bool shared, hipStream_t s, float* d_tran
         reg->r2c_rows(ncl, c->d_sumF, c->d_sumA, c->d_cnt, occ_from(c), c->d_tw_N, c->d_spec2,
                       s);
     } else if (reg) {
-      reg->r2c(ncl, c->d_sumI, c->d_sumR, c->d_cnt, c->d_row_occ, false, c->d_tw_N, c->d_spec, s);
+      reg->r2c(ncl, c->d_sumI, c->d_sumR, c->d_cnt, c->d_row_occ, c->d_tw_N, c->d_spec, s);
       if (four)
-        reg->r2c(ncl, c->d_sumF, c->d_sumA, c->d_cnt, c->d_row_occ, false, c->d_tw_N, c->d_spec2,
-                 s);
+        reg->r2c(ncl, c->d_sumF, c->d_sumA, c->d_cnt, c->d_row_occ, c->d_tw_N, c->d_spec2, s);
     } else {
       const uint8_t* rows = lds_occ ? c->d_row_occ : nullptr;
       launch_spatial_r2c(N, ncl, c->d_sumI, c->d_sumR, c->d_cnt, c->plan_N, c->d_tw_N,
@@ -822,9 +821,11 @@ int spatial_passes(phz_ctx* c, int np, bool shared, hipStream_t s, float* d_tran
         reg->inv_plane(np, c->d_work, c->d_tw_N, d_trans_corr, c->d_partials, slab, s);
       }
       trans_partials = N;
-      if (c->profiling) {  // a stage of its own for the argmax: the pose else does it
+      // every stage has a time: the argmax, which the pose kernel does in
+      // all runs, once more on its own (its keys are not read)
+      if (c->profiling) {
         StageScope t(c, kSpatialC2r, s);
-        launch_reduce_keys(c->d_partials, N, np, c->d_keys + np, s);
+        launch_reduce_keys(c->d_partials, N, np, c->d_keys, s);
       }
     } else {
       {

@@ -308,15 +308,14 @@ struct SpatialReg {
   void (*lines)(int dir, float2* data, int nbatch, int64_t batch_stride, int outer, int inner,
                 const float2* tw, hipStream_t s);
   // r2c of the voxel means; row_occ (nullable: every row read) skips the
-  // empty rows' loads; with sparse_out their (zero) spectrum rows are not
-  // written either, and only x_occ may read the spectra afterwards
+  // empty rows' loads
   void (*r2c)(int nclouds, const float* sumI, const float* sumR, const uint32_t* cnt,
-              const uint8_t* row_occ, bool sparse_out, const float2* tw, float2* spec,
-              hipStream_t s);
+              const uint8_t* row_occ, const float2* tw, float2* spec, hipStream_t s);
   // r2c of the real grids a and b (nullable) into spec and spec + H
   void (*r2c_dense)(const float* a, const float* b, const float2* tw, float2* spec, hipStream_t s);
-  // the sparse r2c over listed occupied rows, one workgroup per z plane (the
-  // same output as r2c with sparse_out)
+  // the sparse r2c: over listed occupied rows, one workgroup or a few per z
+  // plane; the spectrum rows of empty ones (zero) are not written, and only
+  // x_occ may read the spectra afterwards
   void (*r2c_rows)(int nclouds, const float* sumI, const float* sumR, const uint32_t* cnt,
                    VoxelOcc occ, const float2* tw, float2* spec, hipStream_t s);
   // the forward x pass over the spectra of nbatch / 2 clouds left by a

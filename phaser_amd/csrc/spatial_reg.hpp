@@ -14,28 +14,23 @@ namespace {
 // pass 1: rows (z, x) along y, contiguous; R2 threads per row, n2 fastest.
 // kDense: the rows are given as two real channels (a1 may be null: one
 // channel, one spectrum out) instead of sums and counts.
-// A row without points (row_occ 0) is not read: its transform is zero.  With
-// sparse_out it is not written either, and a workgroup whose rows are all
-// empty ends at once.
+// A row without points (row_occ 0) is not read: its transform is zero.
 template <int L, bool kDense>
 __global__ void __launch_bounds__(RegSplit<L>::TPB) k_spat_r2c_reg(
     const float* __restrict__ sumI, const float* __restrict__ sumR,
     const uint32_t* __restrict__ cnt, int64_t cloud_stride, const uint8_t* __restrict__ row_occ,
-    bool sparse_out, const float2* __restrict__ tw, float2* __restrict__ spec,
-    int64_t spec_stride0, int64_t spec_stride1) {
+    const float2* __restrict__ tw, float2* __restrict__ spec, int64_t spec_stride0,
+    int64_t spec_stride1) {
   constexpr int R1 = RegSplit<L>::R1, R2 = RegSplit<L>::R2, LINES = RegSplit<L>::LINES, S = RegSplit<L>::kRowStride;
   constexpr int h = L / 2 + 1;
   __shared__ float2 buf[LINES * S];
   __shared__ float2 table[L];
-  __shared__ uint8_t row_live[LINES];
   const int ln = threadIdx.x / R2, n2 = threadIdx.x % R2;
   const int row0 = blockIdx.x * LINES, c = blockIdx.y;
   const int nrow = L * L - row0 < LINES ? L * L - row0 : LINES;  // of this workgroup
   const uint8_t* occ = row_occ ? row_occ + (int64_t)c * L * L + row0 : nullptr;
   const bool live = ln < nrow && (!occ || occ[ln]);
   const LdsTwiddles<L> w = stage_twiddles<L>(table, n2, tw);
-  if (n2 == 0) row_live[ln] = live;  // read after the transform's barriers
-  if (sparse_out && !__syncthreads_or(live)) return;  // uniform over the workgroup
   const int64_t off = c * cloud_stride + (int64_t)(row0 + ln) * L;
   float2 v[R1];
   if (kDense && live) {
@@ -75,7 +70,6 @@ __global__ void __launch_bounds__(RegSplit<L>::TPB) k_spat_r2c_reg(
   float2* o1 = o0 + spec_stride1;
   for (int idx = threadIdx.x; idx < nrow * h; idx += blockDim.x) {
     const int r = idx / h, k = idx - r * h;
-    if (sparse_out && !row_live[r]) continue;
     const float2 zk = buf[r * S + k];
     const float2 zc = cconj(buf[r * S + (L - k) % L]);
     const float2 sm = cadd(zk, zc), d = csub(zk, zc);
@@ -175,7 +169,7 @@ __global__ void __launch_bounds__(RegSplit<L>::TPB) k_spat_r2c_rows(
   }
 }
 
-// Forward x pass over the spectra a sparse_out r2c left (spectrum b of
+// Forward x pass over the spectra a sparse r2c left (spectrum b of
 // cloud b / 2, layout [z][x][k2], k2 < h = L/2+1): line q = (z, k2) along x
 // (stride h).  When plane z holds no points the line is zero and is neither
 // read nor written; otherwise row x is read only where row (z, x) holds
@@ -693,17 +687,15 @@ struct SpatialRegT {
       hipLaunchKernelGGL((k_fft_lines<+1, L>), g, dim3(TPB), 0, s, data, batch_stride, nl, inner, tw);
   }
   static void r2c(int nclouds, const float* sumI, const float* sumR, const uint32_t* cnt,
-                  const uint8_t* row_occ, bool sparse_out, const float2* tw, float2* spec,
-                  hipStream_t s) {
+                  const uint8_t* row_occ, const float2* tw, float2* spec, hipStream_t s) {
     hipLaunchKernelGGL((k_spat_r2c_reg<L, false>), dim3((L * L + LINES - 1) / LINES, nclouds),
-                       dim3(TPB), 0, s, sumI, sumR, cnt, T, row_occ, sparse_out, tw, spec, 2 * H,
-                       H);
+                       dim3(TPB), 0, s, sumI, sumR, cnt, T, row_occ, tw, spec, 2 * H, H);
   }
   static void r2c_dense(const float* a, const float* b, const float2* tw, float2* spec,
                         hipStream_t s) {
     hipLaunchKernelGGL((k_spat_r2c_reg<L, true>), dim3((L * L + LINES - 1) / LINES, 1), dim3(TPB),
-                       0, s, a, b, (const uint32_t*)nullptr, T, (const uint8_t*)nullptr, false, tw,
-                       spec, (int64_t)0, b ? H : (int64_t)-1);
+                       0, s, a, b, (const uint32_t*)nullptr, T, (const uint8_t*)nullptr, tw, spec,
+                       (int64_t)0, b ? H : (int64_t)-1);
   }
   static void r2c_rows(int nclouds, const float* sumI, const float* sumR, const uint32_t* cnt,
                        VoxelOcc occ, const float2* tw, float2* spec, hipStream_t s) {
