@@ -457,14 +457,14 @@ __global__ void __launch_bounds__(256) k_spat_cross_zz(
         if (!entry(i, e, ii)) break;
         const float2 x = R[ii * ls + e];
         float2* a = &acc[ii * ls + e];
-        const bool sum = ((modes >> (2 * i)) & 3u) == 1u;
         if (first) {
-          // a NaN never has the largest energy: it only stays in a sum
-          const float en = x.x * x.x + x.y * x.y;
-          *a = sum || en == en ? x : make_float2(0.f, 0.f);
+          *a = x;
         } else {
+          // the maximum is the first of equal energies, and a number before a NaN
           const float2 y = *a;
-          const bool take = x.x * x.x + x.y * x.y > y.x * y.x + y.y * y.y;
+          const bool sum = ((modes >> (2 * i)) & 3u) == 1u;
+          const float ey = y.x * y.x + y.y * y.y;
+          const bool take = !(fmaxf(ey, x.x * x.x + x.y * x.y) == ey);
           *a = sum ? cadd(y, x) : (take ? x : y);
         }
       }
@@ -484,7 +484,16 @@ __global__ void __launch_bounds__(256) k_spat_cross_zz(
     } else if (m != 0u) {
       f = g = make_float2(0.f, 0.f);
     }
-    A[ii * ls + e] = make_float2(f.x * g.x - f.y * (-g.y), f.x * (-g.y) + f.y * g.x);
+    float2 c = make_float2(f.x * g.x - f.y * (-g.y), f.x * (-g.y) + f.y * g.x);
+    if (c.x != c.x && m == 0u) {  // a side without a channel that is a number is zero
+      const float ef = f.x * f.x + f.y * f.y, eg = g.x * g.x + g.y * g.y;
+      if (ef != ef || eg != eg) {
+        if (ef != ef) f = make_float2(0.f, 0.f);
+        if (eg != eg) g = make_float2(0.f, 0.f);
+        c = make_float2(f.x * g.x - f.y * (-g.y), f.x * (-g.y) + f.y * g.x);
+      }
+    }
+    A[ii * ls + e] = c;
   }
   __syncthreads();
   const float2* R = lds_fft<+1>(A, B, IT, plan, tws, ls);
