@@ -410,8 +410,10 @@ int check_config(const phz_config& cf) {
 }
 
 // A field of 0 is what a new context has.  The register engine wherever it has
-// the length: against the LDS passes, whole calls at B = 64, 128^3 voxels, 16
-// pairs 1.03 against 3.44 ms, one pair 0.32 against 0.44 ms.  No whole-plane
+// the length: whole calls against the LDS passes at B = 32, one pair and 24 M
+// voxels' worth of them, two and four channels, at each of the 20 lengths: 8 to
+// 61% less time (48^3 one pair 166 against 181 us, 128^3 11 pairs 532 / 1152,
+// 256^3 one pair with four channels 518 / 1323).  No whole-plane
 // forward pass: slower at N = 128 (one workgroup per CU).
 void apply_tuning(phz_ctx* c, const phz_tuning& t) {
   c->tuning = t;
@@ -1868,8 +1870,9 @@ int phz_get_tuning(const phz_ctx* c, phz_tuning* t) {
 // The whole translation stage under candidate choices, on a synthetic scan in
 // every cloud slot, as a call at max_batch runs it: an option that suits one
 // pass can cost more in the others (an LDS tile or the plane pass switches the
-// skipping of empty rows and planes off).  A new context's choices stay unless
-// another one is faster by more than two timings of one form differ.
+// skipping of empty rows and planes off).  Only the tiles of dense passes are
+// timed by themselves, as a call runs them too.  A new context's choices stay
+// unless another one is faster by more than two timings of one form differ.
 int phz_autotune(phz_ctx* c, int repeats, phz_tuning* out) {
   PHZ_CHECK(c, "null argument");
   PHZ_CHECK(repeats >= 1 && repeats <= 1000, "repeats out of range");
@@ -1881,42 +1884,56 @@ int phz_autotune(phz_ctx* c, int repeats, phz_tuning* out) {
   const bool profiling = c->profiling;
   int rc = 0;
   hipEvent_t a = nullptr, b = nullptr;
-  // ms of one run of f; the first one is not timed, and one slower than limit
-  // is not repeated
+  // ms of one run of f: the first one is not timed, one slower than limit is
+  // not repeated, else the best of three means (single launches are short
+  // beside the time to queue them)
   auto timed = [&](auto f, float limit) {
-    float ms = 0.f;
+    float best_of = 0.f;
     f();
-    for (int pass = 0; pass < 2 && !rc; ++pass) {
+    for (int block = 0; block < 4 && !rc; ++block) {
+      const int runs = block ? repeats : 1;
+      float ms = 0.f;
       if (hipEventRecord(a, s) != hipSuccess) rc = -2;
-      for (int r = 0; r < (pass ? repeats : 1); ++r) f();
+      for (int r = 0; r < runs; ++r) f();
       if (hipEventRecord(b, s) != hipSuccess || hipEventSynchronize(b) != hipSuccess ||
           hipEventElapsedTime(&ms, a, b) != hipSuccess || hipGetLastError() != hipSuccess)
         rc = -2;
-      if (pass == 0 && ms > limit) return ms;
+      ms /= (float)runs;
+      if (block == 0 && ms > limit) return ms;
+      if (block == 0 || ms < best_of) best_of = ms;
     }
-    return ms / (float)repeats;
+    return best_of;
   };
   AccumulatorUse use(c, s);
   TRY(use.begin());
   {
     // 64 rings of a scanner in the middle of the grid: ground below, walls
-    // around at 0.3 to 0.6 of its half width
+    // around at 0.3 to 0.6 of its half width; the sources turned by 0.6 rad
+    // about y and then z, which spreads the ground over many z planes
     const int n = (int)std::min<int64_t>(c->cap, 65536), ring = std::max(n / 64, 1);
-    std::vector<float> scan((size_t)n * 4);
+    std::vector<float> scan((size_t)n * 4), turned((size_t)n * 4);
+    const float co = std::cos(0.6f), si = std::sin(0.6f);
     const float mid = 0.5f * (c->vox.lo + c->vox.hi), half = 0.5f * (c->vox.hi - c->vox.lo);
     for (int i = 0; i < n; ++i) {
       const float az = 6.2831853f * (float)(i % ring) / (float)ring;
       const float el = -0.44f + 0.7f * (float)(i / ring % 64) / 64.f;
       const float wall = half * (0.45f + 0.15f * std::sin(3.f * az)), low = -0.04f * half;
       const float dist = el < 0.f ? std::min(wall, low / std::tan(el)) : wall;
-      scan[4 * i] = mid + dist * std::cos(az);
-      scan[4 * i + 1] = mid + dist * std::sin(az);
-      scan[4 * i + 2] = mid + dist * std::tan(el);
-      scan[4 * i + 3] = (float)(1 + i % 97);
+      const float x = dist * std::cos(az), y = dist * std::sin(az), z = dist * std::tan(el);
+      const float xt = co * x + si * z, zt = co * z - si * x;
+      const float point[2][3] = {{x, y, z}, {co * xt - si * y, si * xt + co * y, zt}};
+      for (int d = 0; d < 3; ++d) {
+        scan[4 * i + d] = mid + point[0][d];
+        turned[4 * i + d] = mid + point[1][d];
+      }
+      scan[4 * i + 3] = turned[4 * i + 3] = (float)(1 + i % 97);
     }
-    for (int k = 0; k < M; ++k)
-      TRY(load_cloud(c, k, k ? (const float*)c->d_pts : scan.data(), n,
-                     k ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice, s));
+    for (int k = 0; k < M; ++k) {  // targets, then sources
+      const bool first = k % P == 0;
+      const float* from = first ? (k ? turned : scan).data()
+                                : (const float*)(c->d_pts + (int64_t)(k / P) * P * c->cap);
+      TRY(load_cloud(c, k, from, n, first ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice, s));
+    }
     TRY(commit_counts(c, M, s));
     launch_voxel_scatter(c->d_pts, c->d_npts, c->cap, M, nullptr, 0, N, c->d_edges, c->d_sumI,
                          c->d_sumR, c->d_cnt, occ_from(c), s, extra_from(c));
@@ -1931,26 +1948,37 @@ int phz_autotune(phz_ctx* c, int repeats, phz_tuning* out) {
   best.nn_seed = before.nn_seed;
   best.xz_slab = before.xz_slab;
   float best_ms = 1e30f, plane_ms = 0.f;
+  auto whole = [&](const phz_tuning& of, float limit) {
+    apply_tuning(c, of);
+    return timed([&] { spatial_passes(c, P, false, s, c->d_peak_trans, false); }, limit);
+  };
   auto consider = [&](const phz_tuning& next) {
     if (rc) return 0.f;
-    apply_tuning(c, next);
-    const float ms = timed([&] { spatial_passes(c, P, false, s, c->d_peak_trans, false); },
-                           1.5f * best_ms);
+    const float ms = whole(next, 1.5f * best_ms);
     if (!rc && ms < kMargin * best_ms) {
       best = c->tuning;
       best_ms = ms;
     }
     return ms;
   };
-  // the tiles of a site but for the one in use, up to a number of columns
-  auto tiles = [&](int32_t phz_tuning::*site, int most = 64) {
+  // the fastest tile of a dense pass that a call runs by itself, timed by itself
+  auto tiles = [&](int32_t phz_tuning::*site, auto run) {
+    if (rc) return;
     const int now = best.*site;
+    float now_ms = timed([&] { run(now); }, 1e30f);
     for (int it : {kRegisterEngine, 8, 16, 32, 64}) {
-      if (it == now || it > most || !fft_cols_tile_ok(N, it)) continue;
-      t = best;
-      t.*site = it;
-      consider(t);
+      if (rc || it == now || !fft_cols_tile_ok(N, it)) continue;
+      const float ms = timed([&] { run(it); }, 1.5f * now_ms);
+      if (rc || ms >= kMargin * now_ms) continue;
+      best.*site = it;
+      now_ms = ms;
     }
+  };
+  auto column_pass = [&](int site) {
+    return [&, site](int it) {
+      launch_spatial_fft_pass(N, site == 2 ? P : 2 * M, site == 2 ? c->d_work : c->d_spec, site,
+                              it, c->plan_N, c->d_tw_N, s);
+    };
   };
   consider(best);
   if (spatial_reg(N)) {
@@ -1966,13 +1994,26 @@ int phz_autotune(phz_ctx* c, int repeats, phz_tuning* out) {
   // the tiles where the chosen form has such a pass: the register engine's
   // forward passes are not tiled unless the grid is padded
   const bool reg = best.fused_reg > 0;
-  if (!reg || padded) {
-    if (best.plane_fwd < 0) tiles(&phz_tuning::fwd_x);
-    // a z pass of its own, or the fused cross spectrum's 8 or 16 columns
-    if (padded || best.plane_fwd > 0) tiles(&phz_tuning::fwd_z);
-    else if (N <= 128) tiles(&phz_tuning::fwd_z, 8);
+  if (padded) {
+    if (best.plane_fwd < 0) tiles(&phz_tuning::fwd_x, column_pass(0));
+    tiles(&phz_tuning::fwd_z, column_pass(1));
+  } else if (!reg && best.plane_fwd > 0) {
+    tiles(&phz_tuning::fwd_z, column_pass(1));
+  } else if (!reg) {
+    for (int it : {kRegisterEngine, 8, 16, 32, 64}) {
+      if (it == best.fwd_x || !fft_cols_tile_ok(N, it)) continue;
+      t = best;
+      t.fwd_x = it;
+      consider(t);
+    }
+    if (N <= 128) {  // the fused cross spectrum has 16 columns or 8
+      t = best;
+      t.fwd_z = best.fwd_z == 8 ? 16 : 8;
+      consider(t);
+    }
   }
-  if (!padded && !(reg && spatial_reg(N)->inv_plane)) tiles(&phz_tuning::inv_x);
+  if (!padded && !(reg && spatial_reg(N)->inv_plane)) tiles(&phz_tuning::inv_x, column_pass(2));
+  if (!rc) best_ms = whole(best, 1e30f);
   // SO(3) alpha + gamma passes: register engine against LDS kernels
   float so3_ms = 0.f;
   const int B = c->Bo, n = c->no;
@@ -1996,10 +2037,7 @@ int phz_autotune(phz_ctx* c, int repeats, phz_tuning* out) {
   launch_fill_u32((uint32_t*)c->d_work, (size_t)2 * P * c->H, 0u, s);
   for (int site = 0; site < 3 && !rc; ++site) {
     const int it = site == 0 ? best.fwd_x : site == 1 ? best.fwd_z : best.inv_x;
-    pass_ms[site] = timed([&] {
-      launch_spatial_fft_pass(N, site == 2 ? P : 2 * M, site == 2 ? c->d_work : c->d_spec, site,
-                              it, c->plan_N, c->d_tw_N, s);
-    }, 1e30f);
+    pass_ms[site] = timed([&] { column_pass(site)(it); }, 1e30f);
   }
   launch_voxel_clear(c->d_pts, c->d_npts, c->cap, M, nullptr, 0, N, c->d_edges, c->d_sumI,
                      c->d_sumR, c->d_cnt, occ_from(c), s, extra_from(c));

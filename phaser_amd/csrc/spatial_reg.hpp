@@ -356,7 +356,13 @@ __device__ __forceinline__ void fused_side(const ChannelSet& X, int64_t off, uin
 // previous transform, which bounds the registers held.
 // Bound by memory: 16 pairs at L = 128 move 0.49 GB in 139 us, 3.5 TB/s of the
 // copy kernel's 4.5 (the spectra of more than a few pairs do not stay in the
-// cache).  Masked buffer loads and branch-free fusion in place of predicated
+// cache); 64 pairs 2.1 GB at 4.4, 16 at 192 1.7 GB at 3.8, 8 at 256 2.2 GB at 3.7.
+// At 150, 180 and 216 (960 and 576 threads: 128 and 168 registers) and with four
+// channels at 200 the state spills: 53, 1 and 1 registers with two channels,
+// 381, 342 and 409 with four, 126 at 200.  It is still well ahead of the LDS form
+// there (whole calls with that form: 7 pairs at 150 575 against 960 us, with four
+// channels 999 / 1514; 4 at 180 542 / 950 and 966 / 1502; 2 at 216 487 / 1039 and
+// 873 / 1688; 3 at 200 with four 862 / 1496).  Masked buffer loads and branch-free fusion in place of predicated
 // global loads and per-entry branches: 367 -> 263 us at L = 192, 87 -> 62 at 96.
 template <int L, int NCH>
 __global__ void __launch_bounds__(RegSplit<L>::TPB, 2) k_spat_cross_zz_reg(

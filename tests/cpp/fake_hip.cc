@@ -19,10 +19,10 @@ std::map<const void*, void*> g_vars;
 std::string g_log;            // one line per launch, copy and wait
 std::string g_fail;           // part of a kernel's name whose next launch fails
 std::vector<std::pair<std::string, float>> g_cost;  // name part -> ms of a launch
-float g_clock = 0.f;
+double g_clock = 0.0;
 hipError_t g_last = hipSuccess;
 struct Event {
-  float at = 0.f;
+  double at = 0.0;
 };
 struct CallConfig {
   dim3 g, b;
@@ -86,7 +86,7 @@ hipError_t hipLaunchKernel(const void* stub, dim3 g, dim3 b, void**, size_t sh, 
     return result(hipErrorInvalidConfiguration);
   for (const auto& c : g_cost)
     if (name.find(c.first) != std::string::npos) g_clock += c.second;
-  g_clock += 1e-3f;
+  g_clock += 1e-3;
   g_log += name + "\n";
   return hipSuccess;
 }
@@ -191,7 +191,7 @@ hipError_t hipEventRecord(hipEvent_t e, hipStream_t) {
 }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t a, hipEvent_t b) {
-  *ms = ((Event*)b)->at - ((Event*)a)->at;
+  *ms = (float)(((Event*)b)->at - ((Event*)a)->at);
   return hipSuccess;
 }
 
