@@ -1450,11 +1450,17 @@ int phz_voxelize(phz_ctx* c, const float* pts, int64_t P, float* out, float* cou
   PHZ_HIP(hipGetLastError());
   PHZ_HIP(hipStreamSynchronize(s));
   use.end();
-  for (int64_t v = 0; v < c->T3; ++v) {
-    out[v] = k[v] ? sI[v] / (float)k[v] : 0.f;
-    out[c->T3 + v] = k[v] ? sR[v] / (float)k[v] : 0.f;
-    if (counts) counts[v] = (float)k[v];
+  // without branches (the sums of empty voxels are zero; counts fit an int), so
+  // that the loops vectorise: with a branch per voxel and the counts in one loop
+  // the call took 213 or 264 us at 48^3 by how the compiler laid it out
+  const int64_t T = c->T3;
+  for (int64_t v = 0; v < T; ++v) {
+    const float n = (float)std::max((int)k[v], 1);
+    out[v] = sI[v] / n;
+    out[T + v] = sR[v] / n;
   }
+  if (counts)
+    for (int64_t v = 0; v < T; ++v) counts[v] = (float)(int)k[v];
   return 0;
 }
 
